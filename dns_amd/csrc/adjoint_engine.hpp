@@ -108,8 +108,6 @@ template <int N> struct Adjoint {
   // Backward stages of one step from its recording: (lamU, lamS) = adjoints of
   // (U_{n+1}, u_stale') in, adjoints of (U_n, u_stale) out.
   static int backward_stages(dns_ctx *c, AdjWork *w, const double *rec) {
-    static const double a_rk[4] = {1 / 6.0, 1 / 3.0, 1 / 3.0, 1 / 6.0};  // main.c:15
-    static const double b_rk[4] = {0.5, 0.5, 1.0, 0.0};                 // main.c:16
     hipStream_t s = c->stream;
     const Geo g = c->g;
     const double dt = c->dt[0], nu = c->nu[0], kmax = c->kmax, sc = c->invn3;
@@ -118,7 +116,7 @@ template <int N> struct Adjoint {
     const dim3 gxa = gx(), bxa(T * TPP);
     const dim3 gyt((g.nk + T - 1) / T, N), gyf = gx(), by(T * TPP);
     const dim3 gz(N * N / PPW), bz(PPW * TPP);
-    auto stage = [&](int r) { return AdjStage{a_rk[r], b_rk[r], dt, nu, kmax}; };
+    auto stage = [&](int r) { return AdjStage{RK_A[r], RK_B[r], dt, nu, kmax}; };
     c->w_ready = 0;  // W holds the adjoint's partials from here on
     k_adj_xa<N, T><<<gxa, bxa, 0, s>>>(w->lamU, w->lamV, W, g, stage(3), tw);
     DNS_LAUNCHED();

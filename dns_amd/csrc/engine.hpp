@@ -488,8 +488,6 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
     double2 *uhn = (double2 *)c->uhn, *acc = (double2 *)c->acc;
     const cx<R> *tw = twR(c);
     const R invn3 = (R)c->invn3;
-    static const double a_rk[4] = {1 / 6.0, 1 / 3.0, 1 / 3.0, 1 / 6.0};  // main.c:15
-    static const double b_rk[4] = {0.5, 0.5, 1.0, 0.0};                 // main.c:16
     // y passes: paired tiles where a tile row is narrower than a line
     constexpr bool PY = x_tiles_paired<TY, R>(), PYF = x_tiles_paired<TYF, R>();
     const dim3 gy = PY ? dim3(paired_blocks((NF + TY - 1) / TY, N), 1, M) : grid_x(TY, M), by(TY * TPP_Y);
@@ -505,7 +503,7 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
       double2 *ph = (c->capture && st == nsteps - 1) ? (double2 *)c->phat : nullptr;
       for (int rk = 0; rk < 4; rk++) {
         const RoctxRange stage_range(stage_names[rk]);
-        RKParams q{c->nudt, c->kmax, a_rk[rk], b_rk[rk]};
+        RKParams q{c->nudt, RK_A[rk], RK_B[rk]};
         const int sl = DNS_NPASS * rk;
         // pass A of this stage ran fused into the previous stage's E
         // the adjoint's recording of this stage's u and omega (FP64, M = 1)

@@ -96,9 +96,12 @@ __device__ __forceinline__ bool in_box(int i, int n, int nk) { return i < nk || 
 
 struct RKParams {
   const double2 *nudt;  // per member (viscosity, time step)
-  double kmax;
-  double a, b;          // a[rk], b[rk] of main.c:15-16 for this stage
+  double a, b;          // RK_A, RK_B of this stage
 };
+
+// RK4 weights (main.c:15-16): Un+1 = Un + sum a dU_r; U_{r+1} = Un + b dU_r.
+static constexpr double RK_A[4] = {1 / 6.0, 1 / 3.0, 1 / 3.0, 1 / 6.0};
+static constexpr double RK_B[4] = {0.5, 0.5, 1.0, 0.0};
 
 template <typename R> __device__ __forceinline__ cx<R> zero() { return mk<R>((R)0, (R)0); }
 
@@ -754,7 +757,6 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
   }
   const double ky = (double)wave<N>(j), kz = (double)k;
   const double nudt = nu * dt;
-  const bool myz = fabs(ky) < q.kmax && fabs(kz) < q.kmax;
   const float nudtf = (float)nudt, af = (float)q.a, bf = (float)q.b;  // mixed stages 0..2
   // The state values of a batch of positions (all three fields) are loaded
   // together and the next batch's loads are issued before this batch's
@@ -764,36 +766,76 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
   // Ur as stored: stage 0 reads Un (double; mixed: its float copy)
   using URT = std::conditional_t<STAGE == 0 && !MIXED_STATE, double2, cx<SR>>;
   using URS = std::conditional_t<STAGE == 0 && !MIXED_STATE, double, SR>;
+  using ST = std::conditional_t<S64, double2, float2>;
   struct Batch {
     URT ur[3][BC];      // stage state (stage 0: Un)
     double2 un[3][BC];  // FP64 stages 1,2 and mixed stage 3: Un
     float2 unf[3][BC];  // mixed stages 1,2: float copy of Un
     double2 ac[3][BC];  // FP64 stages 1..3: accumulator
-    std::conditional_t<S64, double2, float2> sf[3][BC];  // mixed stages 1..3: running sum S
+    ST sf[3][BC];       // mixed stages 1..3: running sum S
   };
   constexpr int NB = E / BC;
+  // Outside the dealiased box, where 70% of the modes lie, N = 0 and the
+  // stages only diffuse: there the stage state and the accumulator are formed
+  // again from Un (diffuse64, diffuse32) and neither stored nor read, which
+  // takes 40% of the bytes from stages 2 and 3 of this memory-bound pass.
+  // n=512 FP64: stage 1 3.41 -> 2.59 ms, stages 2, 3 4.64 -> 2.96, stage 4
+  // 2.83 -> 2.48, step 33.9 -> 29.4 ms; float stages 2, 3 2.38 -> 1.59, step
+  // 18.7 -> 16.3; n=96 FP64 step 0.387 -> 0.373 ms, mixed 0.287 -> 0.279.  Below n=96
+  // everything stays in the last-level cache and the longer chain of
+  // operations is what shows (n=72: 0.268 -> 0.279 ms, n=64: 0.154 -> 0.159):
+  // those grids store and read all modes.
+  constexpr bool SKIP = N >= 96;
+  auto boxed = [&](int c) { return nl && okn && in_box(t + TPP * c, N, g.nk); };
   auto load = [&](Batch &B, auto BB) {
     constexpr int c0 = decltype(BB)::value * BC;
     if (!ok) return;
 #pragma unroll
     for (int i = 0; i < BC; i++) {
+      const bool in = !SKIP || STAGE == 0 || boxed(c0 + i);
 #pragma unroll
       for (int f = 0; f < 3; f++) {
         const long lf = f * g.fs + srow(jrow + t + TPP * (c0 + i), k, g);
         if constexpr (STAGE == 0 && MIXED_STATE) B.ur[f][i] = ld_state<T>(inc + lf);
         else if constexpr (STAGE == 0) B.ur[f][i] = ld_state<T>(uhn + lf);
-        else B.ur[f][i] = ld_state<T>(uhr + lf);
+        else B.ur[f][i] = in ? ld_state<T>(uhr + lf) : URT{};
         if constexpr (MIXED_STATE) {
           if constexpr (STAGE == 1 || STAGE == 2) B.unf[f][i] = ld_state<T>(inc + lf);
           if constexpr (STAGE == 3) B.un[f][i] = ld_state<T>(uhn + lf);
-          if constexpr (STAGE > 0 && S64) B.sf[f][i] = ld_state<T>(s64 + lf);
-          else if constexpr (STAGE > 0) B.sf[f][i] = ld_state<T>(inc + 3 * g.fs + lf);
+          if constexpr (STAGE > 0 && S64) B.sf[f][i] = in ? ld_state<T>(s64 + lf) : ST{};
+          else if constexpr (STAGE > 0) B.sf[f][i] = in ? ld_state<T>(inc + 3 * g.fs + lf) : ST{};
         } else {
           if constexpr (STAGE == 1 || STAGE == 2) B.un[f][i] = ld_state<T>(uhn + lf);
-          if constexpr (STAGE > 0) B.ac[f][i] = ld_state<T>(acc + lf);
+          if constexpr (STAGE == 1 || STAGE == 2) B.ac[f][i] = in ? ld_state<T>(acc + lf) : double2{};
+          if constexpr (STAGE == 3) B.ac[f][i] = ld_state<T>((in ? acc : uhn) + lf);
         }
       }
     }
+  };
+  // Stage state ur and accumulator (FP64: ac; mixed: the sum S) of a mode
+  // outside the box: the operations of the stages before, in their order,
+  // with du = -(vk ur).
+  auto diffuse64 = [](double2 un, double vk, double2 &ur, double2 &ac) {
+    ur = ac = un;
+    static_for<0, STAGE>([&](auto r) {
+#pragma clang fp contract(off)
+      const double2 du = make_double2(-(vk * ur.x), -(vk * ur.y));
+      ac = make_double2(ac.x + RK_A[r] * du.x, ac.y + RK_A[r] * du.y);
+      ur = make_double2(un.x + RK_B[r] * du.x, un.y + RK_B[r] * du.y);
+    });
+  };
+  auto diffuse32 = [](float2 un, float vk, float2 &ur, ST &s) {
+    ur = un;
+    static_for<0, STAGE>([&](auto r) {
+#pragma clang fp contract(off)
+      const float2 du = make_float2(-(vk * ur.x), -(vk * ur.y));
+      constexpr float b = (float)RK_B[r];
+      constexpr auto a = std::conditional_t<S64, double, float>(RK_A[r]);
+      const ST ad{a * du.x, a * du.y};
+      if constexpr (r == 0) s = ad;
+      else s = ST{s.x + ad.x, s.y + ad.y};
+      ur = make_float2(un.x + b * du.x, un.y + b * du.y);
+    });
   };
   auto apply = [&](const Batch &B, auto BB) {
     constexpr int c0 = decltype(BB)::value * BC;
@@ -805,7 +847,8 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
       const long l = srow(jrow + t + TPP * c, k, g);
       const double kx = (double)wave<N>(t + TPP * c);
       const double kk = kx * kx + ky * ky + kz * kz;
-      const double fac = (myz && fabs(kx) < q.kmax) ? dt : 0.0;
+      const bool box = boxed(c), in = !SKIP || box;
+      const double fac = box ? dt : 0.0;
       if constexpr (MIXED_STATE) {
         // Mixed state: dU is made from the float nonlinear term and the float
         // stage state, so the expressions of main.c:381-399 are evaluated in
@@ -830,13 +873,17 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
 #pragma unroll
         for (int f = 0; f < 3; f++) {
           const long lf = f * g.fs + l;
-          const float2 ur = cvt<float, URS>(B.ur[f][i]);
+          float2 ur = cvt<float, URS>(B.ur[f][i]);
+          ST sa{0, 0};
+          if constexpr (STAGE > 0) {
+            sa = B.sf[f][i];
+            if (!in) diffuse32(STAGE == 3 ? cvt<float, double>(B.un[f][i]) : B.unf[f][i], vkf, ur, sa);
+          }
           e[f].x -= Pf.x * kvf[f] + vkf * ur.x;
           e[f].y -= Pf.y * kvf[f] + vkf * ur.y;
           const float2 du = e[f];
           if constexpr (STAGE == 3) {
             const double2 un = B.un[f][i];
-            const auto sa = B.sf[f][i];
             double2 nn = make_double2(un.x + (double)sa.x, un.y + (double)sa.y);
             nn = make_double2(nn.x + q.a * (double)du.x, nn.y + q.a * (double)du.y);
             st<double>(uhn + lf, nn);
@@ -846,19 +893,18 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
           }
           const float2 un = STAGE == 0 ? ur : B.unf[f][i];
           const float2 nr = make_float2(un.x + bf * du.x, un.y + bf * du.y);
-          st<SR>(uhr + lf, cvt<SR, float>(nr));
+          if (in) st<SR>(uhr + lf, cvt<SR, float>(nr));
           if constexpr (S64) {
             const double2 ad = make_double2(q.a * (double)du.x, q.a * (double)du.y);
             if constexpr (STAGE == 0) {
-              st<double>(s64 + lf, ad);
+              if (in) st<double>(s64 + lf, ad);
             } else {
-              const double2 sa = B.sf[f][i];
-              st<double>(s64 + lf, make_double2(sa.x + ad.x, sa.y + ad.y));
+              if (in) st<double>(s64 + lf, make_double2(sa.x + ad.x, sa.y + ad.y));
             }
           } else {
-            const float2 sa = STAGE == 0 ? make_float2(0.f, 0.f) : B.sf[f][i];
-            st<float>(inc + 3 * g.fs + lf,
-                      STAGE == 0 ? make_float2(af * du.x, af * du.y) : make_float2(sa.x + af * du.x, sa.y + af * du.y));
+            if (in)
+              st<float>(inc + 3 * g.fs + lf, STAGE == 0 ? make_float2(af * du.x, af * du.y)
+                                                        : make_float2(sa.x + af * du.x, sa.y + af * du.y));
           }
           nxt[f] = cvt<R, float>(nr);
         }
@@ -881,24 +927,26 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
 #pragma unroll
         for (int f = 0; f < 3; f++) {
           const long lf = f * g.fs + l;
-          const double2 ur = cvt<double, URS>(B.ur[f][i]);
+          double2 ur = cvt<double, URS>(B.ur[f][i]), ac;
+          if constexpr (STAGE > 0) {
+            ac = B.ac[f][i];
+            if (!in) diffuse64(STAGE == 3 ? ac : B.un[f][i], vk, ur, ac);
+          }
           d[f].x -= P.x * kv[f] + vk * ur.x;
           d[f].y -= P.y * kv[f] + vk * ur.y;
           const double2 du = d[f];
           if constexpr (STAGE == 0) {
             const cx<SR> nr = cvt<SR, double>(make_double2(ur.x + q.b * du.x, ur.y + q.b * du.y));
-            st<SR>(uhr + lf, nr);
-            st<double>(acc + lf, make_double2(ur.x + q.a * du.x, ur.y + q.a * du.y));
+            if (in) st<SR>(uhr + lf, nr);
+            if (in) st<double>(acc + lf, make_double2(ur.x + q.a * du.x, ur.y + q.a * du.y));
             nxt[f] = cvt<R, SR>(nr);
           } else if constexpr (STAGE < 3) {
             const double2 un = B.un[f][i];
             const cx<SR> nr = cvt<SR, double>(make_double2(un.x + q.b * du.x, un.y + q.b * du.y));
-            st<SR>(uhr + lf, nr);
-            const double2 ac = B.ac[f][i];
-            st<double>(acc + lf, make_double2(ac.x + q.a * du.x, ac.y + q.a * du.y));
+            if (in) st<SR>(uhr + lf, nr);
+            if (in) st<double>(acc + lf, make_double2(ac.x + q.a * du.x, ac.y + q.a * du.y));
             nxt[f] = cvt<R, SR>(nr);
           } else {
-            const double2 ac = B.ac[f][i];
             const double2 nn = make_double2(ac.x + q.a * du.x, ac.y + q.a * du.y);
             st<double>(uhn + lf, nn);
             nxt[f] = cvt<R, double>(nn);

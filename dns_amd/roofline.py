@@ -10,12 +10,15 @@ spectral field and Rr = n^3 reals per physical field:
   B     r 3Uc w 3Uc             r 5Uc w 6Uc               as 2,3
   C     r 3Uc+3Rr w 3Zc         r 6Uc w 3Zc               r 6Uc w 3Zc+3Rr
   D     r 3Zc w 3Yc             as 1                      as 1
-  E     r 3Yc+3Uc(f64)          r 3Yc+3Uc(SR)+6Uc(f64)    r 3Yc+3Uc(SR)+3Uc(f64)
-        w 3Uc(SR)+3Uc(f64)      w 3Uc(SR)+3Uc(f64)        w 3Uc(f64)
+  E     r 3Yc+3Uc(f64)          r 3Yc+3Bc(SR)+3Bc+3Uc     r 3Yc+3Bc(SR)+3Uc(f64)
+        w 3Bc(SR)+3Bc(f64)      w 3Bc(SR)+3Bc(f64)        w 3Uc(f64)
         (FP64; the mixed-precision state terms are listed in slot_bytes)
 
-where Zc = n^2 nk and Yc = n (2nk-1) nk count the dealiased part of the
-nonlinear term (nk = #{m >= 0 : m < kmax}, kmax = 2/3 (n/2+1)).  From stage 2
+where Zc = n^2 nk, Yc = n (2nk-1) nk and Bc = (2nk-1)^2 nk count the
+dealiased part of the nonlinear term after z, y and x (nk = #{m >= 0 : m <
+kmax}, kmax = 2/3 (n/2+1)).  Outside that box the modes only diffuse, and E
+forms the stage state and the accumulator from the step's first state: they
+are stored and read inside it only.  From stage 2
 on, A hands u, v, w, omega_y, omega_z to B, which forms omega_x from v and w
 (5 fields read, 6 written) -- except in FP64 where a y pencil needs more
 than 64 threads at the schedule's elements per thread (n=1024): there A
@@ -24,7 +27,7 @@ writes all six fields and B reads six.
 Partials (A..E outputs) and the stale velocity are in the working precision
 R; the step-start state and the accumulator are always double; SR is the
 stage state's precision (= R).  A step at n=512 (A fused into the previous
-stage's E) moves 171.2 GB in FP64 and 92.1 GB in mixed precision.
+stage's E) moves 146.3 GB in FP64 and 78.5 GB in mixed precision.
 """
 
 PEAK_HBM_GBS = 8000.0  # MI355X HBM3E, published peak
@@ -71,6 +74,7 @@ def slot_bytes(n, precision="fp64"):
     nk = n_box(n)
     zc = n * n * nk                # after the z pass, kz < kmax
     yc = n * (2 * nk - 1) * nk     # after the y pass, also |ky| < kmax
+    bc = (2 * nk - 1) ** 2 * nk    # the dealiased box
     r = 8 if precision == "fp64" else 4      # real scalar in the working precision
     cr, csr, c64 = 2 * r, 2 * r, 16
     out = {}
@@ -86,21 +90,21 @@ def slot_bytes(n, precision="fp64"):
             c = 6 * uc * cr + 3 * zc * cr + 3 * rr * r
         d = 3 * zc * cr + 3 * yc * cr
         if precision == "fp64":
-            if st == 0:
-                e = 3 * yc * cr + 3 * uc * c64 + 3 * uc * csr + 3 * uc * c64
-            elif st < 3:
-                e = 3 * yc * cr + 3 * uc * csr + 6 * uc * c64 + 3 * uc * csr + 3 * uc * c64
-            else:
-                e = 3 * yc * cr + 3 * uc * csr + 3 * uc * c64 + 3 * uc * c64
+            if st == 0:    # r Un; w Ur, acc
+                e = 3 * yc * cr + 3 * uc * c64 + 3 * bc * csr + 3 * bc * c64
+            elif st < 3:   # r Un, Ur, acc; w Ur, acc
+                e = 3 * yc * cr + 3 * uc * c64 + 6 * bc * csr + 6 * bc * c64
+            else:          # r Ur and acc, Un outside the box; w Un+1
+                e = 3 * yc * cr + 3 * bc * csr + 3 * uc * c64 + 3 * uc * c64
         else:  # float copy of Un and running sum S (float; double in mixed_acc64); Un, Un+1 double
             c32 = 8
             cs = c64 if precision == "mixed_acc64" else c32
             if st == 0:    # r Un copy; w Ur(SR), S
-                e = 3 * yc * cr + 3 * uc * c32 + 3 * uc * csr + 3 * uc * cs
-            elif st < 3:   # r Ur, Un copy, S; w Ur, S
-                e = 3 * yc * cr + 3 * uc * csr + 3 * uc * c32 + 3 * uc * cs + 3 * uc * csr + 3 * uc * cs
+                e = 3 * yc * cr + 3 * uc * c32 + 3 * bc * csr + 3 * bc * cs
+            elif st < 3:   # r Un copy, Ur, S; w Ur, S
+                e = 3 * yc * cr + 3 * uc * c32 + 6 * bc * csr + 6 * bc * cs
             else:          # r Ur, Un(f64), S; w Un+1(f64) and its float copy
-                e = 3 * yc * cr + 3 * uc * csr + 3 * uc * c64 + 3 * uc * cs + 3 * uc * c64 + 3 * uc * c32
+                e = 3 * yc * cr + 3 * bc * csr + 3 * uc * c64 + 3 * bc * cs + 3 * uc * c64 + 3 * uc * c32
         # E fused with the next stage's A: A's writes without its read
         nxt_writes = 3 * uc * cr if st == 3 else ax * uc * cr
         for p, v in zip(PASSES, (a, b, c, d, e, e + nxt_writes)):
