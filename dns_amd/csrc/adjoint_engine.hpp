@@ -51,8 +51,8 @@ struct AdjWork {
 
 template <int N> struct Adjoint {
   static constexpr int E = Sched<N>::E, TPP = N / E;
-  static constexpr int T = 8 * TPP > 512 ? 512 / TPP : 8;
-  static constexpr int PPW = z_pencils_per_block<N>();
+  static constexpr int T = tile_cols(8, TPP, 512);
+  static constexpr int PPW = z_pencils_per_block<N, double>();
   static constexpr int NF = N / 2 + 1;
   static dim3 gx() { return dim3((NF + T - 1) / T, N); }
 

@@ -208,14 +208,14 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_adj_z(double2 *__res
   double L0[E], L1[E], L2[E];
   {
     double2 z[E];
-    herm_pair<N, double>(z, w, w + g.wfs, t, g.nk);
+    herm_pair<N, double, z_in_wave<N, PPW>()>(z, w, w + g.wfs, t, g.nk);
     fft_pencil<N, double, true>(z, t, lds, slot, tw);
 #pragma unroll
     for (int c = 0; c < E; c++) {
       L0[c] = z[c].x;
       L1[c] = z[c].y;
     }
-    herm_pair<N, double>(z, w + 2 * g.wfs, nullptr, t, g.nk);
+    herm_pair<N, double, z_in_wave<N, PPW>()>(z, w + 2 * g.wfs, nullptr, t, g.nk);
     fft_pencil<N, double, true>(z, t, lds, slot, tw);
 #pragma unroll
     for (int c = 0; c < E; c++) L2[c] = z[c].x;

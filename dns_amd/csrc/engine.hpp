@@ -221,21 +221,23 @@ namespace dnsk {
 template <int N, typename R, typename SR, bool S64 = false> struct Engine final : Impl {
   static constexpr int E = Sched<N>::E, TPP = N / E;
   // Column tiles of the strided passes: 128-byte row segments (8 double /
-  // 16 float columns).  Blocks holding double state or the fused x pass
-  // have at most 512 threads (256 registers per thread, no spills at
-  // n=1024); the float x pass gets its 16 columns in 512 threads with 16
-  // elements per thread where the schedule allows (powers of two from 256
-  // on); float y passes use up to 1024 threads.
-  static constexpr int T_D = 8 * TPP > 512 ? 512 / TPP : 8;
+  // 16 float columns), or the largest power of two of columns that fits the
+  // block (tiles of 6 or 10 columns split lines unevenly between blocks:
+  // n=576 mixed x pass 31.5 -> 11.8 ms a step with 8).  Blocks holding double
+  // state or the fused x pass have at most 512 threads (256 registers per
+  // thread, no spills at n=1024); float y passes use up to 1024.
+  static constexpr int T_D = tile_cols(8, TPP, 512);
   // y passes: double grids whose pencils need more than 64 threads (n=1024)
   // take 16 elements per thread, keeping 8-column tiles in 512 threads
   // (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
   static constexpr int E_Y = (sizeof(R) == 8 && TPP > 64 && N % (2 * E) == 0) ? 2 * E : E;
   static constexpr int TPP_Y = N / E_Y;
   // 8 double / 16 float columns (float y passes use up to 1024 threads;
-  // narrower float tiles over-fetch: 64-byte segments read 1.8x their bytes)
-  static constexpr int T_Y = sizeof(R) == 8 ? (8 * TPP_Y > 512 ? 512 / TPP_Y : 8)
-                                            : (16 * TPP_Y > 1024 ? 1024 / TPP_Y : 16);
+  // narrower float tiles over-fetch: 64-byte segments read 1.8x their bytes).
+  // Above 768 threads a thread has 128 registers, which 12 or more elements
+  // exceed (n=648 mixed, 272 bytes of spills: y passes 24.3 ms a step against
+  // 15.9 with 8 columns; 9 elements still gain, n=486 7.3 -> 5.9).
+  static constexpr int T_Y = tile_cols(sizeof(R) == 8 ? 8 : 16, TPP_Y, E_Y <= 9 ? 1024 : 768);
   static constexpr int T_YF = T_Y;
   // fields loaded ahead: inverse y pass two in float (1.47 -> 1.38 ms at
   // n=512), one in double (a second costs occupancy), none with 16-element
@@ -252,21 +254,22 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // (348 bytes; 16.1 -> 21.5 ms), so the x pass transforms and stores curlX
   static constexpr bool CX_IN_Y = !(sizeof(R) == 8 && E_Y > E);
   // plain transforms of the working precision (rfft3 / irfft3)
-  static constexpr int T_P = sizeof(R) == 8 ? T_D : (16 * TPP > 1024 ? 1024 / TPP : 16);
-  static constexpr int E_X = (sizeof(R) == 4 && E == 8 && N >= 256) ? 16 : E;
+  static constexpr int T_P = sizeof(R) == 8 ? T_D : tile_cols(16, TPP, 1024);
+  // x pass: 16 float elements per thread give 16-column tiles in fewer threads
+  // (a whole step of six n=192 members: 6.10 -> 5.95 ms)
+  static constexpr int E_X = (sizeof(R) == 4 && E == 8 && N >= 192) ? 16 : E;
   static constexpr int TPP_X = N / E_X;
   // Epilogue batching of the x pass, stages 1-3 (EPI_X) and 4 (EPI_X3): the
   // float epilogue of the mixed state leaves room for four positions per
   // load batch with 16-element threads (n=512: 1.94 -> 1.86 ms in stage 1,
   // 2.66 -> 2.64 in stages 2-3, 2.99 -> 2.95 in stage 4; prefetching the
-  // next batch instead costs more).  The double epilogue keeps the default.
-  static constexpr int EPI_X = (sizeof(SR) == 4 && E_X == 16) ? 4 : 0;
+  // next batch instead costs more), and for three with 9 (n=486: 8.22 -> 7.95
+  // ms a step).  The double epilogue keeps the default.
+  static constexpr int EPI_X = sizeof(SR) == 8 ? 0 : E_X == 16 ? 4 : E_X == 9 ? 3 : 0;
   static constexpr int EPI_X3 = EPI_X;
-  static constexpr int T_X = sizeof(R) == 8 ? T_D : (16 * TPP_X > 512 ? 512 / TPP_X : 16);
-  // z pencils per block: at most one wave (or one pencil when a pencil needs
-  // more than a wave), so the pass's barriers never couple independent
-  // pencils across waves.
-  static constexpr int PPW = z_pencils_per_block<N>();
+  static constexpr int T_X = tile_cols(sizeof(R) == 8 ? 8 : 16, TPP_X, 512);
+  // z pencils per block, of the working precision and of the double passes
+  static constexpr int PPW = z_pencils_per_block<N, R>(), PPW64 = z_pencils_per_block<N, double>();
   static constexpr int NF = N / 2 + 1;
   // recording kernels exist for FP64 only (the adjoint's precision)
   static constexpr bool REC_OK = sizeof(R) == 8;
@@ -275,10 +278,13 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // (at most 128 VGPRs instead of 136-152, spilling at most 28 bytes per
   // lane), 0.982 -> 0.911 ms per launch at n=512 and 0.128 -> 0.119 ms at
   // n=256 in alternating same-box runs.  Not with 12 or 6 elements per
-  // thread (the radix-3 grids), where that bound spills 84-616 and up to 72
-  // bytes per lane.  FP64 keeps 1 (n=1024: 2 spills 92-124 bytes per lane
-  // in stages 2-4 and measured no faster, 20.4 against 20.0-20.2 ms).
-  static constexpr int MINW_Z = (sizeof(R) == 4 && TPP <= 64 && E == 8) ? 4 : 1;
+  // thread, where that bound spills 84-616 and up to 72 bytes per lane.
+  // Nine elements: 3 in float (n=486: 5.80 -> 4.65 ms a step) and 2 in FP64
+  // (12.3 -> 10.1), 3 there spilling far too much (28.7).  Otherwise FP64
+  // keeps 1 (n=1024: 2 spills 92-124 bytes per lane in stages 2-4 and
+  // measured no faster, 20.4 against 20.0-20.2 ms; n=576, 12 elements: 17.0
+  // -> 36.1 ms a step with 2).
+  static constexpr int MINW_Z = sizeof(R) == 4 ? (E == 9 ? 3 : E == 8 && TPP <= 64 ? 4 : 1) : E == 9 ? 2 : 1;
 
   size_t sr_size() const override { return sizeof(cx<SR>); }
   // bytes per member of the accumulator region: 3 double fields, or in
@@ -350,7 +356,7 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
     // physical input is dead by then), then copied into uhn
     double2 *uh = (double2 *)c->uhn + m * c->g.mS;
     double2 *ws = (double2 *)wslice(c, m);
-    k_zr2c<N, double, PPW><<<N * N / PPW, PPW * TPP, 0, s>>>(tmp, uh, 3, c->g, twD(c));
+    k_zr2c<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP, 0, s>>>(tmp, uh, 3, c->g, twD(c));
     DNS_LAUNCHED();
     k_ypass<N, double, T_D, false><<<grid_x(T_D), T_D * TPP, 0, s>>>(uh, 3, c->g, twD(c));
     DNS_LAUNCHED();
@@ -414,8 +420,8 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   static constexpr int T_YFH = T_YF >= 4 ? T_YF / 2 : T_YF;
   static constexpr int T_XH = T_X >= 4 ? T_X / 2 : T_X;
   // two waves of pencils; where a wave's pencils do not fill it exactly
-  // (64 % TPP != 0) a second set would straddle the wave boundary, which the
-  // lane exchanges of the Hermitian loads do not allow: one set only
+  // (64 % TPP != 0) a second set would straddle the wave boundary: one set
+  // only
   static constexpr int PPW2 = (TPP > 64 || 64 % TPP == 0) && (N * N) % (2 * PPW) == 0 ? 2 * PPW : PPW;
   int variants() const override { return TUNABLE ? 4 : 1; }
 
@@ -561,7 +567,7 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
     DNS_LAUNCHED();
     k_ypass<N, double, T_D, true><<<grid_x(T_D), T_D * TPP, 0, s>>>(tmpc, 1, c->g, twD(c));
     DNS_LAUNCHED();
-    k_zc2r<N, double, PPW><<<N * N / PPW, PPW * TPP, 0, s>>>(tmpc, phys, c->g, scale, twD(c));
+    k_zc2r<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP, 0, s>>>(tmpc, phys, c->g, scale, twD(c));
     DNS_LAUNCHED();
     return DNS_OK;
   }

@@ -53,14 +53,41 @@ struct Geo {
   long wfs, wps;
 };
 
-// z pencils per block of the contiguous-axis passes: as many as fill one
-// wave (one pencil when a pencil needs a wave or more), reduced to a divisor
-// of the n*n rows so that every block is full.
-template <int N> constexpr int z_pencils_per_block() {
-  constexpr int TPP = N / Sched<N>::E;
+// z pencils per block of the contiguous-axis passes: as many as fill one wave
+// (one pencil when it needs a wave or more), reduced to a divisor of the n*n
+// rows so that every block is full.  Pencils of threes can leave a quarter of
+// that wave or more idle (48 threads, or two of 24); the smallest count that
+// fills up to three waves then takes its place where the registers leave
+// room for such blocks: at most 6 elements per thread, or a single float
+// pencil.  z passes of a step: n=96 FP64 98 -> 91 us, n=288 FP64 1.93 -> 1.56
+// ms, n=384 mixed 2.78 -> 2.28, n=432 mixed 4.07 -> 3.65.  It loses with 8 or
+// 9 double elements (n=384 FP64 3.86 -> 4.27, n=432 7.13 -> 7.36) and with
+// two float pencils of 8 (six n=192 members: 5.98 -> 6.10 ms a step), and
+// blocks of five to eight waves lose anywhere (n=324 FP64 2.74 -> 4.01).
+template <int N, typename R> constexpr int z_pencils_per_block() {
+  constexpr int E = Sched<N>::E, TPP = N / E;
   int p = TPP >= 64 ? 1 : 64 / TPP;
   while ((N * N) % p) p--;
+  if (TPP < 64 && 4 * p * TPP <= 3 * 64 && (E <= 6 || (sizeof(R) == 4 && p == 1))) {
+    for (int q = p + 1; q * TPP <= 192; q++)
+      if ((N * N) % q == 0 && q * TPP % 64 == 0) return q;
+  }
   return p;
+}
+// Whether every pencil of a block of PPW pencils lies within one wave, so
+// that its lanes can exchange values.
+template <int N, int PPW> constexpr bool z_in_wave() {
+  constexpr int TPP = N / Sched<N>::E;
+  return TPP <= 64 && (PPW * TPP <= 64 || 64 % TPP == 0);
+}
+
+// Columns of a strided pass's tile: a power of two, so that tiles cut the
+// 128-byte lines of a row evenly, at most `want`, in at most `threads`
+// threads of tpp per pencil.
+constexpr int tile_cols(int want, int tpp, int threads) {
+  int t = want;
+  while (t > 1 && t * tpp > threads) t /= 2;
+  return t;
 }
 
 // Column tile (bx) and row (by) of a strided-pass block.  Tiles whose rows
@@ -232,7 +259,7 @@ __global__ __launch_bounds__(T *(N / E), MINW) void k_ypass(cx<R> *__restrict__ 
 #pragma unroll
         for (int c = 0; c < E; c++) {  // I*(ky w - kz v), I*z = (-Im z, Re z)
           const R ky = (R)wave<N>(t + TPP * c);
-          ox[c] = mk<R>(-(ky * v[c].y - ox[c].y), ky * v[c].x - ox[c].x);
+          ox[c] = mk<R>(fm(-ky, v[c].y, ox[c].y), fm(ky, v[c].x, -ox[c].x));
         }
       }
     }
@@ -310,26 +337,27 @@ __device__ __forceinline__ void curl_inverse_x(cx<R> (&U)[E], cx<R> (&V)[E], cx<
       for (int c = 0; c < E; c++) st<R>(W + f * g.wfs + off + (t + TPP * c) * istr, v[c]);
     }
   };
-  auto irot = [](R a, R b) { return mk<R>(-b, a); };  // I*(a + i b)
+  // I*(a p - b q)
+  auto icurl = [](R a, cx<R> p, R b, cx<R> q) { return mk<R>(fm(-a, p.y, b * q.y), fm(a, p.x, -(b * q.x))); };
   {
     cx<R> v[E];
     if constexpr (!WITH_U || CX) {
 #pragma unroll
-      for (int c = 0; c < E; c++) v[c] = irot(ky * Wv[c].x - kz * V[c].x, ky * Wv[c].y - kz * V[c].y);  // curlX
+      for (int c = 0; c < E; c++) v[c] = icurl(ky, Wv[c], kz, V[c]);  // curlX
       fft_pencil<N, R, true>(v, t, lds, slot, tw);
       store(3, v);
     }
 #pragma unroll
     for (int c = 0; c < E; c++) {  // curlY = I*(kz U - kx W)
       const R kx = (R)wave<N>(t + TPP * c);
-      v[c] = irot(kz * U[c].x - kx * Wv[c].x, kz * U[c].y - kx * Wv[c].y);
+      v[c] = icurl(kz, U[c], kx, Wv[c]);
     }
     fft_pencil<N, R, true>(v, t, lds, slot, tw);
     store(4, v);
 #pragma unroll
     for (int c = 0; c < E; c++) {  // curlZ = I*(kx V - ky U)
       const R kx = (R)wave<N>(t + TPP * c);
-      v[c] = irot(kx * V[c].x - ky * U[c].x, kx * V[c].y - ky * U[c].y);
+      v[c] = icurl(kx, V[c], ky, U[c]);
     }
     fft_pencil<N, R, true>(v, t, lds, slot, tw);
     store(5, v);
@@ -396,44 +424,53 @@ template <typename R> __device__ __forceinline__ cx<R> lane_get(cx<R> v, int src
     return mk<R>(get(v.x), get(v.y));
   }
 }
-template <int N, typename R>
+template <int N, typename R, bool IN_WAVE>
 __device__ __forceinline__ void herm_load(HermRaw<N, R> &h, const cx<R> *X, const cx<R> *Y, int t,
                                           int lim = N / 2 + 1) {
   constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
   // Coefficients k >= lim are taken as zero and not read.
-  if constexpr (TPP <= 64) {
+  if constexpr (IN_WAVE) {
     // Each stored element is loaded once (non-temporal): positions pos <= H
-    // directly (pos < H sit at c < E/2: t + TPP c < TPP E/2 = H); pos > H
-    // needs k = N - pos = TPP (E - c) - t, which thread TPP - t of the same
-    // pencil (same wave) holds at index E - 1 - c (for t = 0: its own index
-    // E - c, or the Nyquist element at c = E/2), passed between lanes.
+    // directly; pos > H needs k = N - pos = TPP (E - c) - t, which thread
+    // TPP - t of the same pencil (same wave) holds at index E - 1 - c (thread
+    // 0: its own index E - c), passed between lanes.  E even: H = TPP E/2, so
+    // c < E/2 is direct and the Nyquist element is thread 0's at c = E/2.  E
+    // odd (TPP even): H falls in the middle of index c = E/2, direct for
+    // t <= TPP/2.
+    constexpr bool ODD = E % 2 != 0;
+    constexpr int MID = E / 2;
 #pragma unroll
-    for (int c = 0; c < E / 2; c++) {
-      const bool in = t + TPP * c < lim;
+    for (int c = 0; c < (E + 1) / 2; c++) {
+      const bool in = t + TPP * c < lim && (!ODD || c < MID || t <= TPP / 2);
       h.x[c] = in ? ldnt(X + t + TPP * c) : zero<R>();
       h.y[c] = Y && in ? ldnt(Y + t + TPP * c) : zero<R>();
     }
     cx<R> nx = zero<R>(), ny = zero<R>();
-    if (t == 0 && H < lim) {
+    if (!ODD && t == 0 && H < lim) {
       nx = ldnt(X + H);
       if (Y) ny = ldnt(Y + H);
     }
     const int lane = (int)(threadIdx.x & 63);
     const int src = lane - t + (TPP - t) % TPP;
 #pragma unroll
-    for (int c = E / 2; c < E; c++) {
+    for (int c = MID; c < E; c++) {
       const cx<R> mx = lane_get<R>(h.x[E - 1 - c], src);
       const cx<R> my = lane_get<R>(h.y[E - 1 - c], src);
-      if (t == 0) {
-        h.x[c] = c == E / 2 ? nx : h.x[E - c];
-        h.y[c] = c == E / 2 ? ny : h.y[E - c];
+      if (ODD && c == MID) {
+        if (t > TPP / 2) {
+          h.x[c] = mx;
+          h.y[c] = my;
+        }
+      } else if (t == 0) {
+        h.x[c] = c == MID ? nx : h.x[E - c];
+        h.y[c] = c == MID ? ny : h.y[E - c];
       } else {
         h.x[c] = mx;
         h.y[c] = my;
       }
     }
   } else {
-    // a pencil over several waves: each thread loads its mirrored positions
+    // a pencil across waves: each thread loads its mirrored positions
     // too, with ordinary loads, so that the second fetch of an element finds
     // it in L2 (the pencil's other half-wave loaded it)
 #pragma unroll
@@ -457,11 +494,11 @@ __device__ __forceinline__ void herm_combine(cx<R> (&z)[Sched<N>::E], const Herm
     else z[c] = mk<R>(x.x + y.y, y.x - x.y);
   }
 }
-template <int N, typename R>
+template <int N, typename R, bool IN_WAVE>
 __device__ __forceinline__ void herm_pair(cx<R> (&z)[Sched<N>::E], const cx<R> *X, const cx<R> *Y, int t,
                                           int lim = N / 2 + 1) {
   HermRaw<N, R> h;
-  herm_load<N, R>(h, X, Y, t, lim);
+  herm_load<N, R, IN_WAVE>(h, X, Y, t, lim);
   herm_combine<N, R>(z, h, t);
 }
 
@@ -508,7 +545,7 @@ template <int N, typename R> __device__ __forceinline__ const cx<R> *z_twiddles(
 // (N_x, N_y) stored; N_z returned in nz.  Loads one Hermitian pair at a
 // time (register budget).  MODE 1, 2: h holds the raw loads of the row's
 // first pair (W fields 0, 1) on entry.
-template <int N, typename R, int MODE, typename UR, bool REC = false>
+template <int N, typename R, int MODE, typename UR, bool IW, bool REC = false>
 __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr, Geo g, R invn3,
                                      const cx<R> *__restrict__ tw, int t, cx<R> *lds, PencilSlot<N> slot,
                                      const R (&oz0)[Sched<N>::E], R (&nz)[Sched<N>::E], const HermRaw<N, R> &h,
@@ -524,7 +561,7 @@ __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr
       v[c] = (R)usr[g.rs + l];
       ww[c] = (R)usr[2 * g.rs + l];
     }
-    herm_pair<N, R>(z1, w + 3 * g.wfs, w + 4 * g.wfs, t);
+    herm_pair<N, R, IW>(z1, w + 3 * g.wfs, w + 4 * g.wfs, t);
     fft_pencil<N, R, true>(z1, t, lds, slot, z_twiddles<N, R>(tw));
 #pragma unroll
     for (int c = 0; c < E; c++) {
@@ -536,9 +573,9 @@ __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr
     cx<R> z1[E], z2[E], z3[E];
     herm_combine<N, R>(z1, h, t);
     fft_pencil<N, R, true>(z1, t, lds, slot, z_twiddles<N, R>(tw));
-    herm_pair<N, R>(z2, w + 2 * g.wfs, w + 3 * g.wfs, t);
+    herm_pair<N, R, IW>(z2, w + 2 * g.wfs, w + 3 * g.wfs, t);
     fft_pencil<N, R, true>(z2, t, lds, slot, z_twiddles<N, R>(tw));
-    herm_pair<N, R>(z3, w + 4 * g.wfs, w + 5 * g.wfs, t);
+    herm_pair<N, R, IW>(z3, w + 4 * g.wfs, w + 5 * g.wfs, t);
     fft_pencil<N, R, true>(z3, t, lds, slot, z_twiddles<N, R>(tw));
 #pragma unroll
     for (int c = 0; c < E; c++) {
@@ -574,8 +611,8 @@ __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr
   cx<R> f1[E];
 #pragma unroll
   for (int c = 0; c < E; c++) {
-    f1[c] = mk<R>(v[c] * oz[c] - ww[c] * oy[c], ww[c] * ox[c] - u[c] * oz[c]);
-    nz[c] = u[c] * oy[c] - v[c] * ox[c];
+    f1[c] = mk<R>(fm(v[c], oz[c], -(ww[c] * oy[c])), fm(ww[c], ox[c], -(u[c] * oz[c])));
+    nz[c] = fm(u[c], oy[c], -(v[c] * ox[c]));
   }
   fft_pencil<N, R, false>(f1, t, lds, slot, z_twiddles<N, R>(tw));
   split_store<N, R>(f1, w, w + g.wfs, t, lds, slot, g.nk);
@@ -599,6 +636,7 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E), MINW) void k_zfused(cx<R> *
                                                                     const cx<R> *__restrict__ tw,
                                                                     double *__restrict__ rec = nullptr) {
   constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+  constexpr bool IW = z_in_wave<N, PPW>();
   __shared__ cx<R> lds[PPW * padlen<N>()];
   const int p = threadIdx.x / TPP, t = threadIdx.x % TPP;
   const long row = (long)blockIdx.x * PPW + p;
@@ -609,14 +647,14 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E), MINW) void k_zfused(cx<R> *
   HermRaw<N, R> h;
   if constexpr (MODE == 0) {
     cx<R> z[E];
-    herm_pair<N, R>(z, w + 5 * g.wfs, nullptr, t);
+    herm_pair<N, R, IW>(z, w + 5 * g.wfs, nullptr, t);
     fft_pencil<N, R, true>(z, t, lds, slot, z_twiddles<N, R>(tw));
 #pragma unroll
     for (int c = 0; c < E; c++) oz0[c] = z[c].x * invn3;
   } else {
-    herm_load<N, R>(h, w, w + g.wfs, t);
+    herm_load<N, R, IW>(h, w, w + g.wfs, t);
   }
-  zrow<N, R, MODE, UR, REC>(w, us + row * N, g, invn3, tw, t, lds, slot, oz0, nz, h,
+  zrow<N, R, MODE, UR, IW, REC>(w, us + row * N, g, invn3, tw, t, lds, slot, oz0, nz, h,
                             REC ? rec + row * N : nullptr);
   // N_z is the transform of a real pencil: its first half is the r2c output.
   cx<R> f2[E];
@@ -675,7 +713,7 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zc2r(const cx<R> *__
   const long row = (long)blockIdx.x * PPW + p;
   const PencilSlot<N> slot{p * padlen<N>()};
   cx<R> z[E];
-  herm_pair<N, R>(z, in + row * g.nfp, nullptr, t);
+  herm_pair<N, R, z_in_wave<N, PPW>()>(z, in + row * g.nfp, nullptr, t);
   fft_pencil<N, R, true>(z, t, lds, slot, tw);
 #pragma unroll
   for (int c = 0; c < E; c++) st_real<double>(out + row * N + t + TPP * c, (double)(z[c].x * scale));
@@ -722,7 +760,7 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
   // two positions per batch (six or nine loads; one position for
   // 16-element threads), next batch prefetched in float tiles of up to 8
   // elements (register budget)
-  constexpr int BC = EPI ? (EPI & 63) : E >= 16 ? 1 : 2;
+  constexpr int BC = EPI ? (EPI & 63) : E >= 16 || E % 2 ? 1 : 2;
   constexpr bool PF = EPI ? (EPI & 64) != 0 : sizeof(R) == 4 && E < 16;
   static_assert(E % BC == 0, "batch must divide the elements per thread");
   W += blockIdx.z * g.mW;
@@ -818,7 +856,6 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
   auto diffuse64 = [](double2 un, double vk, double2 &ur, double2 &ac) {
     ur = ac = un;
     static_for<0, STAGE>([&](auto r) {
-#pragma clang fp contract(off)
       const double2 du = make_double2(-(vk * ur.x), -(vk * ur.y));
       ac = make_double2(ac.x + RK_A[r] * du.x, ac.y + RK_A[r] * du.y);
       ur = make_double2(un.x + RK_B[r] * du.x, un.y + RK_B[r] * du.y);
@@ -827,7 +864,6 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
   auto diffuse32 = [](float2 un, float vk, float2 &ur, ST &s) {
     ur = un;
     static_for<0, STAGE>([&](auto r) {
-#pragma clang fp contract(off)
       const float2 du = make_float2(-(vk * ur.x), -(vk * ur.y));
       constexpr float b = (float)RK_B[r];
       constexpr auto a = std::conditional_t<S64, double, float>(RK_A[r]);

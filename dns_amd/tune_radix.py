@@ -14,7 +14,9 @@ a few percent between processes with where its buffers land in device
 memory.  Every candidate must also reproduce the table schedule's result to
 rounding (energy and enstrophy after the timed steps within 1e-12
 relative; the spectral state within 1e-11 of its max norm up to n=256).
-The chosen schedules are entered in the table by hand.
+The chosen schedules are entered in the table by hand.  Sizes with a
+DNS_SCHED_WIDE entry (radices up to 16, a middle one that need not divide E)
+run that one; the tuner still starts from their DNS_SCHED entry.
 
     python -m dns_amd.tune_radix build 128 256     # on the CPU: dns_amd/_tune/
     python -m dns_amd.tune_radix run 128 256       # on the GPU: one JSON line per candidate
