@@ -29,6 +29,7 @@
 #include <vector>
 #include "../../include/dns.h"
 #include "kernels.hpp"
+#include "plane_fused.hpp"
 
 namespace dnsk {
 
@@ -52,6 +53,7 @@ struct Impl;
 
 // Kernel timing slots: DNS_NPASS * stage + pass; passes 0..4 = A..E of
 // kernels.hpp, 5 = E fused with the next stage's A.
+// (where k_plane runs B, C and D in one launch it is timed as C)
 enum { DNS_NPASS = 6, DNS_NSLOT = 4 * DNS_NPASS };
 
 struct dns_ctx {
@@ -227,6 +229,17 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // state or the fused x pass have at most 512 threads (256 registers per
   // thread, no spills at n=1024); float y passes use up to 1024.
   static constexpr int T_D = tile_cols(8, TPP, 512);
+  // Passes B, C and D in one launch, one block per x-plane (k_plane), where
+  // that is faster than three launches over the whole chip: double up to
+  // n=48, float up to n=72.  Microseconds a step, three launches -> one: FP64
+  // n=8 79 -> 50, n=16 80 -> 55, n=32 98 -> 81, n=48 131 -> 121, but n=54 147
+  // -> 160 and n=64 147 -> 209 (a plane's transforms keep one CU busy, and
+  // three quarters of the chip idle); mixed n=16 71 -> 50, n=32 98 -> 71,
+  // n=48 123 -> 98, n=64 129 -> 125, n=72 165 -> 151, six n=64 members 351 ->
+  // 322.  At n=64 the columns of two fields and 4 elements per thread would
+  // take 1056 threads.
+  static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
+  static constexpr int E_P = N == 64 ? 2 * E : E;
   // y passes: double grids whose pencils need more than 64 threads (n=1024)
   // take 16 elements per thread, keeping 8-column tiles in 512 threads
   // (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
@@ -514,7 +527,21 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
         // pass A of this stage ran fused into the previous stage's E
         // the adjoint's recording of this stage's u and omega (FP64, M = 1)
         double *rp = (sizeof(R) == 8 && c->rec_phys) ? c->rec_phys + (size_t)rk * 6 * g.rs : nullptr;
-        if (rk == 0) {
+        if constexpr (PLANE) {
+          const dim3 gp(N, 1, M), bp(Plane<N, E_P>::THREADS);
+          if (rp && rk == 0)
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+          else if (rp && rk < 3)
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+          else if (rp)
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+          else if (rk == 0)
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+          else if (rk < 3)
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+          else
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+        } else if (rk == 0) {
           DNS_TIMED(c, sl + 1, (k_ypass<N, R, TY, true, 1, PIPE_Y, false, E_Y, false, true, PY><<<gy, by, 0, s>>>(W + 3 * g.wfs, 3, g, tw, g.mW)));
           if (rp)
             DNS_TIMED(c, sl + 2, (k_zfused<N, R, PP, 0, R, MINW_Z, REC_OK><<<gz, bz, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
@@ -534,8 +561,9 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
           else
             DNS_TIMED(c, sl + 2, (k_zfused<N, R, PP, 2, R, MINW_Z><<<gz, bz, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
         }
-        DNS_TIMED(c, sl + 3,
-                  (k_ypass<N, R, TYF, false, 1, PIPE_YF, true, E_Y, false, true, PYF><<<gy_trunc, byf, 0, s>>>(W, 3, g, tw, g.mW)));
+        if constexpr (!PLANE)
+          DNS_TIMED(c, sl + 3,
+                    (k_ypass<N, R, TYF, false, 1, PIPE_YF, true, E_Y, false, true, PYF><<<gy_trunc, byf, 0, s>>>(W, 3, g, tw, g.mW)));
         // E fused with the next stage's A (the next step's stage 1 after rk 3)
         switch (rk) {
           case 0:

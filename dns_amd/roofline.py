@@ -74,6 +74,12 @@ def curlx_in_y(n, precision="fp64"):
     return not wide
 
 
+def plane_fused(n, precision="fp64"):
+    """Whether one launch runs B, C and D on whole x-planes (Engine::PLANE of
+    csrc/engine.hpp); it is timed as zfused."""
+    return n <= (48 if precision == "fp64" else 72)
+
+
 def slot_bytes(n, precision="fp64"):
     """{slot name: algorithmic bytes of one launch}; slot = pass.s<stage>.
 
@@ -100,6 +106,8 @@ def slot_bytes(n, precision="fp64"):
         else:
             c = 6 * uc * cr + 3 * zc * cr + 3 * rr * r
         d = 3 * zc * cr + 3 * yc * cr
+        if plane_fused(n, precision):  # the partials between B, C and D stay in LDS
+            b, c, d = 0, c - 3 * zc * cr + 3 * yc * cr - (0 if st == 0 else (6 - ax) * uc * cr), 0
         if precision == "fp64":
             if st == 0:    # r Un; w Ur, acc
                 e = 3 * yc * cr + 3 * uc * c64 + 3 * bc * csr + 3 * bc * c64

@@ -136,7 +136,8 @@ int dns_autotune(dns_ctx *ctx, int steps, int *best_shape);
  * by HIP events on the context's stream; times accumulate per slot
  * 6*stage + pass (stage 0..3; pass 0..5 = x-inverse with curl, y-inverse,
  * fused z pass, y-forward, x-forward with the RK update, and x-forward with
- * the RK update fused with the next stage's x-inverse).  Switching on or off
+ * the RK update fused with the next stage's x-inverse).  Small grids run
+ * passes 1 to 3 in one launch, timed as pass 2.  Switching on or off
  * resets the sums.  dns_kernel_timing synchronises and fills
  * ms[DNS_KERNEL_SLOTS] and launches[DNS_KERNEL_SLOTS]; dns_kernel_slot_name
  * gives "<pass>.s<stage 1..4>". */
