@@ -240,9 +240,9 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // take 1056 threads.
   static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
   static constexpr int E_P = N == 64 ? 2 * E : E;
-  // y passes: double grids whose pencils need more than 64 threads (n=1024)
-  // take 16 elements per thread, keeping 8-column tiles in 512 threads
-  // (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
+  // y passes: double grids whose pencils need more than 64 threads (n=864 to
+  // 1024) take twice the elements per thread (n=1024: 16), keeping 8-column
+  // tiles in 512 threads (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
   static constexpr int E_Y = (sizeof(R) == 8 && TPP > 64 && N % (2 * E) == 0) ? 2 * E : E;
   static constexpr int TPP_Y = N / E_Y;
   // 8 double / 16 float columns (float y passes use up to 1024 threads;
@@ -287,7 +287,7 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // recording kernels exist for FP64 only (the adjoint's precision)
   static constexpr bool REC_OK = sizeof(R) == 8;
   // minimum waves per SIMD the z pass's registers must allow.  Float with 8
-  // elements per thread and a pencil in at most one wave (n = 32..512): 4
+  // elements per thread and a pencil in at most one wave: 4
   // (at most 128 VGPRs instead of 136-152, spilling at most 28 bytes per
   // lane), 0.982 -> 0.911 ms per launch at n=512 and 0.128 -> 0.119 ms at
   // n=256 in alternating same-box runs.  Not with 12 or 6 elements per

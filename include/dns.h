@@ -51,7 +51,7 @@ enum {
  *            energy/enstrophy reductions are double.
  * DNS_MIXED_ACC64: as DNS_MIXED, but the running sum S of the stage
  *            increments is formed and stored in double (FP64 RK4
- *            accumulation; 3 more float fields of device memory and 10.5%
+ *            accumulation; 3 more float fields of device memory and 3.7%
  *            more bytes per step at n=512). */
 enum dns_precision { DNS_FP64 = 0, DNS_MIXED = 1, DNS_MIXED_ACC64 = 2 };
 
