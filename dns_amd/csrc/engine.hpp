@@ -261,7 +261,11 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // array and loads no field ahead: in float two ahead spill at 1024
   // threads and one leaves a small spill (1.14 against 1.13 ms at n=512);
   // in double one ahead costs 192 against 160 VGPRs (2.51 against 2.47 ms)
-  static constexpr int PIPE_YC = 0;
+  // -- except where an FP64 block has fewer than 512 threads and at most 9
+  // elements, whose registers allow it (inverse y passes of a step, none -> one
+  // ahead: n=216 710 -> 683 us, n=288 1612 -> 1516, n=384 3665 -> 3347, n=486
+  // 7098 -> 6613; below n=216 no difference)
+  static constexpr int PIPE_YC = sizeof(R) == 8 && E_Y <= 9 && T_Y * TPP_Y < 512 && N >= 216 ? 1 : 0;
   // curlX formed by the inverse y pass, except where that pass runs 16
   // double elements per thread (n=1024): there its extra array spills
   // (348 bytes; 16.1 -> 21.5 ms), so the x pass transforms and stores curlX
@@ -292,12 +296,13 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // lane), 0.982 -> 0.911 ms per launch at n=512 and 0.128 -> 0.119 ms at
   // n=256 in alternating same-box runs.  Not with 12 or 6 elements per
   // thread, where that bound spills 84-616 and up to 72 bytes per lane.
+  // Blocks of three waves: 3 (n=384 mixed, z passes of a step 2.63 -> 2.17 ms).
   // Nine elements: 3 in float (n=486: 5.80 -> 4.65 ms a step) and 2 in FP64
   // (12.3 -> 10.1), 3 there spilling far too much (28.7).  Otherwise FP64
   // keeps 1 (n=1024: 2 spills 92-124 bytes per lane in stages 2-4 and
   // measured no faster, 20.4 against 20.0-20.2 ms; n=576, 12 elements: 17.0
   // -> 36.1 ms a step with 2).
-  static constexpr int MINW_Z = sizeof(R) == 4 ? (E == 9 ? 3 : E == 8 && TPP <= 64 ? 4 : 1) : E == 9 ? 2 : 1;
+  static constexpr int MINW_Z = sizeof(R) == 4 ? (E == 9 || PPW * TPP == 192 ? 3 : E == 8 && TPP <= 64 ? 4 : 1) : E == 9 ? 2 : 1;
 
   size_t sr_size() const override { return sizeof(cx<SR>); }
   // bytes per member of the accumulator region: 3 double fields, or in
