@@ -16,10 +16,10 @@ spectral field and Rr = n^3 reals per physical field:
 
 where Zc = n^2 nk, Yc = n (2nk-1) nk and Bc = (2nk-1)^2 nk count the
 dealiased part of the nonlinear term after z, y and x (nk = #{m >= 0 : m <
-kmax}, kmax = 2/3 (n/2+1)).  Outside that box the modes only diffuse, and E
-forms the stage state and the accumulator from the step's first state: they
-are stored and read inside it only.  From stage 2
-on, A hands u, v, w, omega_y, omega_z to B, which forms omega_x from v and w
+kmax}, kmax = 2/3 (n/2+1)).  Outside that box the modes only diffuse, and from
+n=96 on (stores_all_modes) E forms the stage state and the accumulator there
+from the step's first state: they are stored and read inside it only.  Smaller
+grids store and read all modes: Uc in the place of Bc.  From stage 2 on, A hands u, v, w, omega_y, omega_z to B, which forms omega_x from v and w
 (5 fields read, 6 written) -- except in FP64 where a y pencil needs more
 than 64 threads at the schedule's elements per thread (n=1024): there A
 writes all six fields and B reads six.
@@ -80,6 +80,12 @@ def plane_fused(n, precision="fp64"):
     return n <= (48 if precision == "fp64" else 72)
 
 
+def stores_all_modes(n):
+    """Whether the x pass stores and reads its stage state and accumulator
+    outside the dealiased box too (SKIP of csrc/kernels.hpp)."""
+    return n < 96
+
+
 def slot_bytes(n, precision="fp64"):
     """{slot name: algorithmic bytes of one launch}; slot = pass.s<stage>.
 
@@ -91,7 +97,8 @@ def slot_bytes(n, precision="fp64"):
     nk = n_box(n)
     zc = n * n * nk                # after the z pass, kz < kmax
     yc = n * (2 * nk - 1) * nk     # after the y pass, also |ky| < kmax
-    bc = (2 * nk - 1) ** 2 * nk    # the dealiased box
+    # modes of the stage state and accumulator: the dealiased box, or all
+    bc = uc if stores_all_modes(n) else (2 * nk - 1) ** 2 * nk
     r = 8 if precision == "fp64" else 4      # real scalar in the working precision
     cr, csr, c64 = 2 * r, 2 * r, 16
     out = {}
@@ -113,7 +120,7 @@ def slot_bytes(n, precision="fp64"):
                 e = 3 * yc * cr + 3 * uc * c64 + 3 * bc * csr + 3 * bc * c64
             elif st < 3:   # r Un, Ur, acc; w Ur, acc
                 e = 3 * yc * cr + 3 * uc * c64 + 6 * bc * csr + 6 * bc * c64
-            else:          # r Ur and acc, Un outside the box; w Un+1
+            else:          # r Ur, and acc or (outside the box) Un; w Un+1
                 e = 3 * yc * cr + 3 * bc * csr + 3 * uc * c64 + 3 * uc * c64
         else:  # float copy of Un and running sum S (float; double in mixed_acc64); Un, Un+1 double
             c32 = 8
