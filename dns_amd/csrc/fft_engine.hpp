@@ -106,10 +106,24 @@ template <typename R> __device__ __forceinline__ void st_real(R *p, R v) {
 
 // ---------------------------------------------------------------------------
 // Radix schedules.  E = elements per thread, so a pencil takes N/E threads.
-// SchedTable holds, for every size, a schedule whose radices all divide E:
-// the fastest of the orderings timed by dns_amd/tune_radix.py (one build per
-// candidate); a build may replace one size's schedule with -DDNS_SCHED_N=n
-// -DDNS_SCHED_E=e -DDNS_SCHED_R=r0,r1,... (the tuner's candidate builds).
+// The first and last radix divide E; a middle one need not (fft_pencil).  E
+// and the number of stages were chosen by hand from builds of one size,
+// the radix order of the power-of-two grids from 128 on by
+// dns_amd/tune_radix.py, which times the other orders of a size against the row
+// below (a candidate build replaces it with -DDNS_SCHED_N=n -DDNS_SCHED_E=e
+// -DDNS_SCHED_R=r0,r1,...).
+//
+// Each stage costs an exchange through LDS and two barriers, and 12
+// elements per thread are what held most grids with a factor 3 back: the
+// FP64 z pass then takes all 512 registers (one wave per SIMD) and the x pass
+// spills.  Microseconds a step of the former 12- and 6-element schedules of
+// radices 4, 3, 2 -> these (one box): FP64 n=96 390 -> 290, n=216 3970 -> 2800,
+// n=432 35600 -> 21600, n=486 58300 -> 29900; mixed n=162 903 -> 752, n=384
+// 9560 -> 8050, n=648 119200 -> 46500, n=972 376700 -> 174000.  Measured
+// and not taken: n=486 and n=648 with 6 elements (28.1 and 63.6 ms mixed:
+// tiles of 4 columns), n=576 8-9-8 (61.7 ms FP64 against 56.1, mixed
+// 33.6 against 28.6), n=128 and n=256 with radix 16 (683 against 573 us, 3.99
+// against 3.74 ms FP64).
 template <int N> struct SchedTable;
 #define DNS_SCHED(N_, E_, ...)                                \
   template <> struct SchedTable<N_> {                         \
@@ -121,72 +135,35 @@ DNS_SCHED(8, 4, 4, 2)
 DNS_SCHED(12, 6, 6, 2)
 DNS_SCHED(16, 4, 4, 4)
 DNS_SCHED(18, 6, 6, 3)
-DNS_SCHED(24, 12, 4, 2, 3)
+DNS_SCHED(24, 4, 4, 3, 2)
 DNS_SCHED(32, 4, 4, 2, 4)
 DNS_SCHED(36, 6, 6, 6)
-DNS_SCHED(48, 12, 4, 4, 3)
+DNS_SCHED(48, 4, 4, 3, 4)
 DNS_SCHED(54, 6, 6, 3, 3)
 DNS_SCHED(64, 4, 4, 4, 4)
 DNS_SCHED(72, 6, 6, 2, 6)
-DNS_SCHED(96, 12, 4, 2, 4, 3)
+DNS_SCHED(96, 4, 4, 6, 4)
 DNS_SCHED(108, 6, 6, 3, 6)
 DNS_SCHED(128, 8, 8, 8, 2)
-DNS_SCHED(144, 12, 12, 12)
-DNS_SCHED(162, 6, 6, 3, 3, 3)
-DNS_SCHED(192, 12, 4, 4, 3, 4)
+DNS_SCHED(144, 6, 6, 4, 6)
+DNS_SCHED(162, 6, 6, 9, 3)
+DNS_SCHED(192, 8, 8, 3, 8)
 DNS_SCHED(216, 6, 6, 6, 6)
 DNS_SCHED(256, 8, 8, 4, 8)
-DNS_SCHED(288, 12, 12, 2, 12)
-DNS_SCHED(324, 6, 6, 3, 3, 6)
-DNS_SCHED(384, 12, 4, 4, 4, 2, 3)
-DNS_SCHED(432, 12, 12, 3, 12)
-DNS_SCHED(486, 6, 6, 3, 3, 3, 3)
+DNS_SCHED(288, 6, 6, 8, 6)
+DNS_SCHED(324, 6, 6, 9, 6)
+DNS_SCHED(384, 8, 8, 6, 8)
+DNS_SCHED(432, 9, 9, 16, 3)
+DNS_SCHED(486, 9, 9, 6, 9)
 DNS_SCHED(512, 8, 8, 8, 8)
 DNS_SCHED(576, 12, 12, 4, 12)
-DNS_SCHED(648, 12, 12, 3, 3, 6)
-DNS_SCHED(768, 12, 4, 4, 4, 4, 3)
+DNS_SCHED(648, 12, 12, 9, 6)
+DNS_SCHED(768, 12, 12, 16, 4)
 DNS_SCHED(864, 12, 12, 6, 12)
-DNS_SCHED(972, 12, 12, 3, 3, 3, 3)
+DNS_SCHED(972, 9, 9, 12, 9)
 DNS_SCHED(1024, 8, 8, 8, 4, 4)
 #undef DNS_SCHED
-// Schedules with a middle radix that does not divide E, for the sizes where
-// one beats the table above: fewer stages (each costs an exchange through
-// LDS and two barriers) at fewer elements per thread.  12 elements per
-// thread are what held most grids with a factor 3 back: the FP64 z pass then
-// takes all 512 registers (one wave per SIMD) and the x pass spills.
-// Microseconds a step of the former 12- and 6-element schedules of radices
-// 4, 3, 2 -> now (one box): FP64 n=96 390 -> 290, n=216 3970 -> 2820 (above),
-// n=432 35600 -> 21600, n=486 58300 -> 29900; mixed n=162 903 -> 752, n=384
-// 9560 -> 8050, n=648 119200 -> 46500, n=972 376700 -> 174000.  Measured
-// and not taken: n=486 and n=648 with 6 elements (28.1 and 63.6 ms mixed:
-// tiles of 4 columns), n=576 8-9-8 (61.7 ms FP64 against 56.1, mixed
-// 33.6 against 28.6), n=128 and n=256 with radix 16 (683 against 573 us, 3.99
-// against 3.74 ms FP64).
-template <int N> struct SchedWide {
-  static constexpr int E = 0;
-};
-#define DNS_SCHED_WIDE(N_, E_, ...)                           \
-  template <> struct SchedWide<N_> {                          \
-    static constexpr int E = E_;                              \
-    static constexpr int r[] = {__VA_ARGS__};                 \
-    static constexpr int NS = sizeof(r) / sizeof(r[0]);       \
-  };
-DNS_SCHED_WIDE(24, 4, 4, 3, 2)
-DNS_SCHED_WIDE(48, 4, 4, 3, 4)
-DNS_SCHED_WIDE(96, 4, 4, 6, 4)
-DNS_SCHED_WIDE(144, 6, 6, 4, 6)
-DNS_SCHED_WIDE(162, 6, 6, 9, 3)
-DNS_SCHED_WIDE(192, 8, 8, 3, 8)
-DNS_SCHED_WIDE(288, 6, 6, 8, 6)
-DNS_SCHED_WIDE(324, 6, 6, 9, 6)
-DNS_SCHED_WIDE(384, 8, 8, 6, 8)
-DNS_SCHED_WIDE(432, 9, 9, 16, 3)
-DNS_SCHED_WIDE(486, 9, 9, 6, 9)
-DNS_SCHED_WIDE(648, 12, 12, 9, 6)
-DNS_SCHED_WIDE(768, 12, 12, 16, 4)
-DNS_SCHED_WIDE(972, 9, 9, 12, 9)
-#undef DNS_SCHED_WIDE
-template <int N> struct Sched : std::conditional_t<(SchedWide<N>::E > 0), SchedWide<N>, SchedTable<N>> {};
+template <int N> struct Sched : SchedTable<N> {};
 #ifdef DNS_SCHED_N
 template <> struct Sched<DNS_SCHED_N> {
   static constexpr int E = DNS_SCHED_E;
@@ -358,7 +335,6 @@ template <typename R, int RAD, bool INV> __device__ __forceinline__ void dft(cx<
   else if constexpr (RAD == 8) dft8<R, INV>(a);
   else if constexpr (RAD == 9) dft9<R, INV>(a);
   else if constexpr (RAD == 12) dft_coprime<R, 4, 3, 3, 1, INV>(a);
-  else if constexpr (RAD == 18) dft_coprime<R, 2, 9, 1, 5, INV>(a);
   else {
     static_assert(RAD == 16, "radix");
     dft16<R, INV>(a);
@@ -404,8 +380,8 @@ template <int N, typename R, bool INV, class Slot, int E>
 __device__ __forceinline__ void fft_pencil(cx<R> (&v)[E], int t, cx<R> *lds, Slot slot,
                                            const cx<R> *__restrict__ tw) {
   constexpr int NS = Sched<N>::NS, TPP = N / E;
-  static_assert(N % E == 0 && E % Sched<N>::r[0] == 0 && E % Sched<N>::r[NS - 1] == 0,
-                "E must divide N, and the first and last radix E");
+  static_assert(stage_Ns<N>(NS) == N && N % E == 0 && E % Sched<N>::r[0] == 0 && E % Sched<N>::r[NS - 1] == 0,
+                "the radices multiply to N, E divides N, the first and last radix divide E");
   static_for<0, NS>([&](auto S) {
     constexpr int s = decltype(S)::value;
     constexpr int r = Sched<N>::r[s];

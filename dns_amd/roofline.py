@@ -44,8 +44,8 @@ def n_box(n):
 
 
 def elements_per_thread(n):
-    """Elements per thread E of n's schedule in the tuner's table (DNS_SCHED
-    entries of csrc/fft_engine.hpp)."""
+    """Elements per thread E of n's radix schedule (DNS_SCHED entries of
+    csrc/fft_engine.hpp: a pencil takes n / E threads)."""
     import os
     import re
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "fft_engine.hpp")
@@ -54,22 +54,11 @@ def elements_per_thread(n):
     return table[n]
 
 
-def pencil_elements(n):
-    """Elements per thread of the schedule that the kernels run: the
-    DNS_SCHED_WIDE entry where there is one, else DNS_SCHED's."""
-    import os
-    import re
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "fft_engine.hpp")
-    with open(path) as f:
-        wide = {int(a): int(b) for a, b in re.findall(r"DNS_SCHED_WIDE\((\d+),\s*(\d+)", f.read())}
-    return wide.get(n) or elements_per_thread(n)
-
-
 def curlx_in_y(n, precision="fp64"):
     """Whether the inverse y pass forms omega_x (see the table above): not
     where FP64 y pencils take twice the schedule's elements per thread (a
     pencil over more than 64 threads, when n divides by 2E)."""
-    e = pencil_elements(n)
+    e = elements_per_thread(n)
     wide = precision == "fp64" and n // e > 64 and n % (2 * e) == 0
     return not wide
 

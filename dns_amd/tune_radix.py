@@ -3,9 +3,10 @@
 A schedule (fft_engine.hpp, DNS_SCHED) fixes the elements per thread E and
 the radix of every Stockham stage; it is a compile-time constant of every
 kernel, so each candidate is a separate build.  The candidates of a size n
-are the orderings of every radix multiset (radices from {2, 3, 4, 8}
-dividing the table's E, product n) with the fewest stages: each stage is
-one exchange through LDS.  Each candidate is compiled into a library of that
+are the table's schedule, which the library runs, and the orderings of every
+radix multiset (radices from {2, 3, 4, 6, 8, 9, 12, 16}, product n) with the
+fewest stages, each stage being one exchange through LDS, whose first and
+last radix divide the table's E.  Each candidate is compiled into a library of that
 one size, with the table's schedule replaced through -DDNS_SCHED_N,
 -DDNS_SCHED_E and -DDNS_SCHED_R, and timed on the GPU against the table's
 schedule (FP64 and mixed Taylor-Green steps, default launch shape), each
@@ -14,9 +15,8 @@ a few percent between processes with where its buffers land in device
 memory.  Every candidate must also reproduce the table schedule's result to
 rounding (energy and enstrophy after the timed steps within 1e-12
 relative; the spectral state within 1e-11 of its max norm up to n=256).
-The chosen schedules are entered in the table by hand.  Sizes with a
-DNS_SCHED_WIDE entry (radices up to 16, a middle one that need not divide E)
-run that one; the tuner still starts from their DNS_SCHED entry.
+The chosen schedules are entered in the table by hand; E and a schedule of
+more stages than the fewest are chosen by hand too.
 
     python -m dns_amd.tune_radix build 128 256     # on the CPU: dns_amd/_tune/
     python -m dns_amd.tune_radix run 128 256       # on the GPU: one JSON line per candidate
@@ -48,20 +48,22 @@ def table():
     return out
 
 
+RADICES = (16, 12, 9, 8, 6, 4, 3, 2)  # dft of fft_engine.hpp
+
+
 def candidates(n):
     """Schedules with the table's E and the fewest stages; the table's own
-    schedule first."""
+    schedule first, whatever its number of stages."""
     e, cur = table()[n]
-    radices = [r for r in (8, 4, 3, 2) if e % r == 0]
     best = []
     for stages in range(1, 12):
-        sets = [c for c in itertools.combinations_with_replacement(radices, stages) if math.prod(c) == n]
-        if sets:
-            for c in sets:
-                best.extend(sorted(set(itertools.permutations(c)), reverse=True))
+        for c in itertools.combinations_with_replacement(RADICES, stages):
+            if math.prod(c) == n:
+                best.extend(p for p in sorted(set(itertools.permutations(c)), reverse=True)
+                            if e % p[0] == 0 and e % p[-1] == 0)
+        if best:
             break
-    best = [cur] + [c for c in best if c != cur]
-    return e, best
+    return e, [cur] + [c for c in best if c != cur]
 
 
 def name(n, rad):
