@@ -18,7 +18,9 @@ from numpy_step import inner, r2c, solenoidal_field, step_tlm
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,seed", [(16, 1), (32, 2), (48, 3)])
+# up to 48 the stages are recorded by the plane kernel, above by the z pass: in
+# one wave (54) and in blocks of three waves whose pencils cross them (72, 96)
+@pytest.mark.parametrize("n,seed", [(16, 1), (32, 2), (48, 3), (54, 4), (72, 5), (96, 6)])
 def test_step_dot_product(n, seed):
     rng = np.random.default_rng(seed)
     nu, dt = 0.02, 0.01
