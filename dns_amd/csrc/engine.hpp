@@ -235,9 +235,12 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // n=8 79 -> 50, n=16 80 -> 55, n=32 98 -> 81, n=48 131 -> 121, but n=54 147
   // -> 160 and n=64 147 -> 209 (a plane's transforms keep one CU busy, and
   // three quarters of the chip idle); mixed n=16 71 -> 50, n=32 98 -> 71,
-  // n=48 123 -> 98, n=64 129 -> 125, n=72 165 -> 151, six n=64 members 351 ->
-  // 322.  At n=64 the columns of two fields and 4 elements per thread would
-  // take 1056 threads.
+  // n=48 123 -> 98, n=64 129 -> 125, n=72 165 -> 151.  Batches, which fill the
+  // chip either way, gain as well, from 2 to 48 members: FP64 n=48 six 296 ->
+  // 284, 48 of them 1816 -> 1509; n=24 133 -> 93 and 340 -> 229; mixed n=64 349
+  // -> 321 and 2329 -> 2047, n=72 478 -> 404 and 3224 -> 2776.
+  // At n=64 the columns of two fields and 4 elements per thread would take 1056
+  // threads.
   static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
   static constexpr int E_P = N == 64 ? 2 * E : E;
   // y passes: double grids whose pencils need more than 64 threads (n=864 to
@@ -263,8 +266,10 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // in double one ahead costs 192 against 160 VGPRs (2.51 against 2.47 ms)
   // -- except where an FP64 block has fewer than 512 threads and at most 9
   // elements, whose registers allow it (inverse y passes of a step, none -> one
-  // ahead: n=216 710 -> 683 us, n=288 1612 -> 1516, n=384 3665 -> 3347, n=486
-  // 7098 -> 6613; below n=216 no difference)
+  // ahead: n=216 710 -> 683 us, n=256 1068 -> 1033, n=288 1612 -> 1516, n=384
+  // 3665 -> 3347, n=432 5470 -> 5305, n=486 7098 -> 6613; below n=216 no
+  // difference).  Some float blocks of that kind would gain less (n=288 878 ->
+  // 850, n=432 2712 -> 2588; n=256 530 -> 534) and load none ahead.
   static constexpr int PIPE_YC = sizeof(R) == 8 && E_Y <= 9 && T_Y * TPP_Y < 512 && N >= 216 ? 1 : 0;
   // curlX formed by the inverse y pass, except where that pass runs 16
   // double elements per thread (n=1024): there its extra array spills
@@ -296,7 +301,8 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // lane), 0.982 -> 0.911 ms per launch at n=512 and 0.128 -> 0.119 ms at
   // n=256 in alternating same-box runs.  Not with 12 or 6 elements per
   // thread, where that bound spills 84-616 and up to 72 bytes per lane.
-  // Blocks of three waves: 3 (n=384 mixed, z passes of a step 2.63 -> 2.17 ms).
+  // Blocks of three waves: 3 (n=384 mixed, z passes of a step 2.63 -> 2.17 ms;
+  // n=96, 144 and 288 measure the same with 1).
   // Nine elements: 3 in float (n=486: 5.80 -> 4.65 ms a step) and 2 in FP64
   // (12.3 -> 10.1), 3 there spilling far too much (28.7).  Otherwise FP64
   // keeps 1 (n=1024: 2 spills 92-124 bytes per lane in stages 2-4 and
@@ -431,8 +437,9 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   }
 
   // Launch shapes selectable at run time (all give identical arithmetic):
-  // bit 0 halves the strided passes' column tile, bit 1 doubles the z pass's
-  // pencils per block.  Only grids up to 512 carry the alternatives.
+  // bit 0 halves the strided passes' column tile (the x pass's alone where
+  // k_plane runs the others), bit 1 doubles the z pass's pencils per block.  Only
+  // grids up to 512 carry the alternatives.
   static constexpr bool TUNABLE = N <= 512;
   static constexpr int T_YH = T_Y >= 4 ? T_Y / 2 : T_Y;
   static constexpr int T_YFH = T_YF >= 4 ? T_YF / 2 : T_YF;

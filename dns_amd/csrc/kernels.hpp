@@ -743,7 +743,7 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zc2r(const cx<R> *__
 // Grid (ceil(nf/T), n): blockIdx.y = j.
 // EPI selects the epilogue's batching: 0 = default (below), otherwise
 // BC = EPI & 63 positions per batch and prefetch of the next batch if
-// EPI & 64.  E = elements per thread (a multiple of every radix of N).
+// EPI & 64.  E = elements per thread (a multiple of the first and last radix).
 template <int N, typename R, int T, int STAGE, typename SR, int EPI = 0, int E = Sched<N>::E, bool S64 = false>
 __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR> *__restrict__ uhr,
                                              double2 *__restrict__ uhn, double2 *__restrict__ acc,

@@ -212,7 +212,7 @@ def test_large_beltrami(n, precision, tol):
 
 def test_interleaved_state_rows_round_trip():
     """n=864 keeps its spectral state with x rows interleaved in pairs (a
-    pencil takes 72 threads; x tiles are 7 columns wide).  The state of a
+    pencil takes 72 threads; x tiles are 4 columns wide).  The state of a
     loaded separable field, read back through dns_get_spectral, holds the
     closed-form coefficients at their (i, j, k) positions; written back with
     dns_set_spectral it reads back bitwise; and the device's enstrophy sum,
