@@ -239,10 +239,10 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // chip either way, gain as well, from 2 to 48 members: FP64 n=48 six 296 ->
   // 284, 48 of them 1816 -> 1509; n=24 133 -> 93 and 340 -> 229; mixed n=64 349
   // -> 321 and 2329 -> 2047, n=72 478 -> 404 and 3224 -> 2776.
-  // At n=64 the columns of two fields and 4 elements per thread would take 1056
-  // threads.
+  // Twice the elements per thread where a plane would take more than 1024
+  // threads (float n=64: 66 columns of 16).
   static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
-  static constexpr int E_P = N == 64 ? 2 * E : E;
+  static constexpr int E_P = Plane<N, E>::THREADS > 1024 ? 2 * E : E;
   // y passes: double grids whose pencils need more than 64 threads (n=864 to
   // 1024) take twice the elements per thread (n=1024: 16), keeping 8-column
   // tiles in 512 threads (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
