@@ -187,8 +187,8 @@ static int ctx_set_spectral(dns_ctx *c, int m, const double *uvw_hat) {
   return c->impl->set_spectral(c, m, uvw_hat);
 }
 
-// Time every launch shape of the context for `steps` steps from its
-// current state, keep the fastest, and restore the state.  All shapes give
+// Time every launch shape of the context that differs from the lower ones for
+// `steps` steps from its current state, keep the fastest, and restore the state.  All shapes give
 // bitwise identical results.
 static int ctx_autotune(dns_ctx *c, int steps, int *best_out, double *best_ms) {
   DNS_HIP(hipSetDevice(c->device));
@@ -218,6 +218,7 @@ static int ctx_autotune(dns_ctx *c, int steps, int *best_out, double *best_ms) {
       hip(hipMemcpyAsync(sus, c->us, ub, hipMemcpyDeviceToDevice, c->stream), "hipMemcpyAsync");
     }
     for (int v = 0; v < nv && rc == DNS_OK; v++) {
+      if (!c->impl->distinct(v)) continue;
       c->impl->set_variant(c, v);
       rc = c->impl->step(c, 1);
       if (rc == DNS_OK) hip(hipEventRecord(a, c->stream), "hipEventRecord");

@@ -116,6 +116,8 @@ struct Impl {
   // taken as present (graph capture after prepare()).
   virtual int step(dns_ctx *c, long nsteps) = 0;
   virtual int variants() const = 0;
+  // whether launch shape v launches anything that a lower one does not
+  virtual bool distinct(int v) const = 0;
   virtual int set_variant(dns_ctx *c, int v) = 0;
   virtual int snapshot(dns_ctx *c, int m, double *uvwp) = 0;
   // c2r(U,V,W,P)/n^3 of member 0 into `dst` (device [4][n][n][n] doubles)
@@ -449,6 +451,11 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // only
   static constexpr int PPW2 = (TPP > 64 || 64 % TPP == 0) && (N * N) % (2 * PPW) == 0 ? 2 * PPW : PPW;
   int variants() const override { return TUNABLE ? 4 : 1; }
+  // A bit selects nothing where its two sides are the same: the z bit where
+  // k_plane takes the z pass's place or a second set does not fit.
+  static constexpr int SHAPE_BITS = (T_XH != T_X || (!PLANE && (T_YH != T_Y || T_YFH != T_YF)) ? 1 : 0) |
+                                    (!PLANE && PPW2 != PPW ? 2 : 0);
+  bool distinct(int v) const override { return (v & ~SHAPE_BITS) == 0; }
 
   int step(dns_ctx *c, long nsteps) override {
     int rc = prepare(c);

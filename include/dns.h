@@ -125,8 +125,10 @@ int dns_irfft3(dns_ctx *ctx, const double *spec, double *real);
 /* Launch shapes.  A context's kernels can run with several block shapes
  * (strided-pass column tile width, z-pass pencils per block) that all give
  * bitwise identical results; grids up to 512 carry 4 shapes, larger grids 1.
- * dns_autotune times each shape for `steps` steps from the current state,
- * keeps the fastest and restores the state. */
+ * Where a shape launches what a lower one does (a wider z block that the grid
+ * has no room for, or no z pass of its own on small grids) both are accepted.
+ * dns_autotune times each shape that differs for `steps` steps from the current
+ * state, keeps the fastest and restores the state. */
 int dns_launch_shapes(dns_ctx *ctx);
 int dns_set_launch_shape(dns_ctx *ctx, int shape);
 int dns_get_launch_shape(dns_ctx *ctx);
