@@ -50,7 +50,7 @@ struct AdjWork {
 };
 
 template <int N> struct Adjoint {
-  static constexpr int E = Sched<N>::E, TPP = N / E;
+  static constexpr int E = Sched<N, double>::E, TPP = N / E;
   static constexpr int T = tile_cols(8, TPP, 512);
   static constexpr int PPW = z_pencils_per_block<N, double>();
   static constexpr int NF = N / 2 + 1;

@@ -84,14 +84,14 @@ __device__ __forceinline__ void adj_pre_x(double2 (&d)[3][E], double2 *__restric
 }
 
 // XA of backward stage 3 (no lamNext): grid (ceil(nf/T), n), blockIdx.y = j.
-template <int N, int T, int E = Sched<N>::E>
+template <int N, int T, int E = Sched<N, double>::E>
 __global__ __launch_bounds__(T *(N / E)) void k_adj_xa(const double2 *__restrict__ lamU, double2 *__restrict__ lamV,
                                                        double2 *__restrict__ W, Geo g, AdjStage q,
                                                        const double2 *__restrict__ tw) {
 #pragma clang fp contract(off)
   constexpr int TPP = N / E;
   __shared__ double2 lds[T * padlen<N>()];
-  __shared__ double2 twl[tw_size<N>()];
+  __shared__ double2 twl[tw_size<N, double>()];
   tw = stage_twiddles<N, double>(twl, tw);
   const int p = threadIdx.x % T, t = threadIdx.x / T;
   const int j = blockIdx.y, k = blockIdx.x * T + p;
@@ -112,14 +112,14 @@ __global__ __launch_bounds__(T *(N / E)) void k_adj_xa(const double2 *__restrict
 //  FU   : F_u present (r > 0); F_w in W fields 0..2, F_u in 3..5
 //  FIRST: r == 3, lamUn = lamU + lamUr (else lamUn += lamUr)
 // qn: the parameters of stage r - 1 (a, b, dt, nu, kmax).
-template <int N, int T, bool FU, bool FIRST, bool NEXT, int E = Sched<N>::E>
+template <int N, int T, bool FU, bool FIRST, bool NEXT, int E = Sched<N, double>::E>
 __global__ __launch_bounds__(T *(N / E)) void k_adj_xe(double2 *__restrict__ W, const double2 *__restrict__ lamU,
                                                        double2 *__restrict__ lamUn, double2 *__restrict__ lamV, Geo g,
                                                        AdjStage qn, const double2 *__restrict__ tw) {
 #pragma clang fp contract(off)
   constexpr int TPP = N / E;
   __shared__ double2 lds[T * padlen<N>()];
-  __shared__ double2 twl[tw_size<N>()];
+  __shared__ double2 twl[tw_size<N, double>()];
   tw = stage_twiddles<N, double>(twl, tw);
   const int p = threadIdx.x % T, t = threadIdx.x / T;
   const int j = blockIdx.y, k = blockIdx.x * T + p;
@@ -193,13 +193,13 @@ __global__ __launch_bounds__(T *(N / E)) void k_adj_xe(double2 *__restrict__ W, 
 //  R0: r == 0 (lam_u to lamSout, only lam_w transformed); LS: r == 3 (lamS in).
 // rec: u_r (fields 0..2) and omega_r (3..5), physical, [6][n][n][n].
 template <int N, int PPW, bool R0, bool LS>
-__global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_adj_z(double2 *__restrict__ W,
+__global__ __launch_bounds__(PPW *(N / Sched<N, double>::E)) void k_adj_z(double2 *__restrict__ W,
                                                                    const double *__restrict__ rec,
                                                                    const double *__restrict__ lamS,
                                                                    double *__restrict__ lamSout, Geo g, double sc,
                                                                    const double2 *__restrict__ tw) {
 #pragma clang fp contract(off)
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+  constexpr int E = Sched<N, double>::E, TPP = N / E, H = N / 2;
   __shared__ double2 lds[PPW * padlen<N>()];
   const int p = threadIdx.x / TPP, t = threadIdx.x % TPP;
   const long row = (long)blockIdx.x * PPW + p;
@@ -208,14 +208,14 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_adj_z(double2 *__res
   double L0[E], L1[E], L2[E];
   {
     double2 z[E];
-    herm_pair<N, double, z_in_wave<N, PPW>()>(z, w, w + g.wfs, t, g.nk);
+    herm_pair<N, double, z_in_wave<N, double, PPW>()>(z, w, w + g.wfs, t, g.nk);
     fft_pencil<N, double, true>(z, t, lds, slot, tw);
 #pragma unroll
     for (int c = 0; c < E; c++) {
       L0[c] = z[c].x;
       L1[c] = z[c].y;
     }
-    herm_pair<N, double, z_in_wave<N, PPW>()>(z, w + 2 * g.wfs, nullptr, t, g.nk);
+    herm_pair<N, double, z_in_wave<N, double, PPW>()>(z, w + 2 * g.wfs, nullptr, t, g.nk);
     fft_pencil<N, double, true>(z, t, lds, slot, tw);
 #pragma unroll
     for (int c = 0; c < E; c++) L2[c] = z[c].x;

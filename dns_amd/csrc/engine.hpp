@@ -198,14 +198,14 @@ __global__ void k_convert(const TI *__restrict__ in, TO *__restrict__ out, long 
     out[i] = (TO)in[i];
 }
 
-// Forward twiddles of the radix schedule of N: per stage s, entries
+// Forward twiddles of the radix schedule of N in precision R: per stage s, entries
 // k*(r-1) + m-1 = exp(-2 pi i m k / (Ns r)), computed in long double.
-template <int N> std::vector<long double> twiddles_ld() {
-  std::vector<long double> t(2 * tw_size<N>() + 2, 0.0L);
+template <int N, typename R> std::vector<long double> twiddles_ld() {
+  std::vector<long double> t(2 * tw_size<N, R>() + 2, 0.0L);
   const long double PI = 3.141592653589793238462643383279502884L;
   int off = 0, Ns = 1;
-  for (int s = 0; s < Sched<N>::NS; s++) {
-    const int r = Sched<N>::r[s];
+  for (int s = 0; s < Sched<N, R>::NS; s++) {
+    const int r = Sched<N, R>::r[s];
     for (int k = 0; k < Ns; k++)
       for (int m = 1; m < r; m++) {
         const long double a = 2.0L * PI * (long double)(m * k) / (long double)(Ns * r);
@@ -223,28 +223,27 @@ template <int N> std::vector<long double> twiddles_ld() {
 namespace dnsk {
 
 template <int N, typename R, typename SR, bool S64 = false> struct Engine final : Impl {
-  static constexpr int E = Sched<N>::E, TPP = N / E;
+  static constexpr int E = Sched<N, R>::E, TPP = N / E;
+  static constexpr int TPP64 = N / Sched<N, double>::E;  // of the double passes
   // Column tiles of the strided passes: 128-byte row segments (8 double /
   // 16 float columns), or the largest power of two of columns that fits the
   // block (tiles of 6 or 10 columns split lines unevenly between blocks:
   // n=576 mixed x pass 31.5 -> 11.8 ms a step with 8).  Blocks holding double
   // state or the fused x pass have at most 512 threads (256 registers per
   // thread, no spills at n=1024); float y passes use up to 1024.
-  static constexpr int T_D = tile_cols(8, TPP, 512);
+  static constexpr int T_D = tile_cols(8, TPP64, 512);
   // Passes B, C and D in one launch, one block per x-plane (k_plane), where
   // that is faster than three launches over the whole chip: double up to
   // n=48, float up to n=72.  Microseconds a step, three launches -> one: FP64
   // n=8 79 -> 50, n=16 80 -> 55, n=32 98 -> 81, n=48 131 -> 121, but n=54 147
   // -> 160 and n=64 147 -> 209 (a plane's transforms keep one CU busy, and
   // three quarters of the chip idle); mixed n=16 71 -> 50, n=32 98 -> 71,
-  // n=48 123 -> 98, n=64 129 -> 125, n=72 165 -> 151.  Batches, which fill the
+  // n=48 123 -> 98, n=64 129 -> 118, n=72 165 -> 151.  Batches, which fill the
   // chip either way, gain as well, from 2 to 48 members: FP64 n=48 six 296 ->
-  // 284, 48 of them 1816 -> 1509; n=24 133 -> 93 and 340 -> 229; mixed n=64 349
-  // -> 321 and 2329 -> 2047, n=72 478 -> 404 and 3224 -> 2776.
-  // Twice the elements per thread where a plane would take more than 1024
-  // threads (float n=64: 66 columns of 16).
+  // 284, 48 of them 1816 -> 1509; n=24 133 -> 93 and 340 -> 229; mixed n=72 478
+  // -> 404 and 3224 -> 2776.
   static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
-  static constexpr int E_P = Plane<N, E>::THREADS > 1024 ? 2 * E : E;
+  static_assert(!PLANE || Plane<N, E>::THREADS <= 1024, "a plane's columns fit a block");
   // y passes: double grids whose pencils need more than 64 threads (n=864 to
   // 1024) take twice the elements per thread (n=1024: 16), keeping 8-column
   // tiles in 512 threads (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).
@@ -337,13 +336,10 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   static char *wslice(dns_ctx *c, int m) { return (char *)c->W + (size_t)m * c->g.mW * sizeof(cx<R>); }
 
   int make_twiddles(dns_ctx *c) override {
-    auto t = twiddles_ld<N>();
-    std::vector<double> d(t.size());
-    std::vector<float> f(t.size());
-    for (size_t i = 0; i < t.size(); i++) {
-      d[i] = (double)t[i];
-      f[i] = (float)t[i];  // single rounding from the long double value
-    }
+    const auto td = twiddles_ld<N, double>(), tf = twiddles_ld<N, float>();
+    // single roundings from the long double values
+    const std::vector<double> d(td.begin(), td.end());
+    const std::vector<float> f(tf.begin(), tf.end());
     DNS_HIP(hipMalloc(&c->tw64, d.size() * sizeof(double)));
     DNS_HIP(hipMemcpy(c->tw64, d.data(), d.size() * sizeof(double), hipMemcpyHostToDevice));
     DNS_HIP(hipMalloc(&c->tw32, f.size() * sizeof(float)));
@@ -382,11 +378,11 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
     // physical input is dead by then), then copied into uhn
     double2 *uh = (double2 *)c->uhn + m * c->g.mS;
     double2 *ws = (double2 *)wslice(c, m);
-    k_zr2c<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP, 0, s>>>(tmp, uh, 3, c->g, twD(c));
+    k_zr2c<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP64, 0, s>>>(tmp, uh, 3, c->g, twD(c));
     DNS_LAUNCHED();
-    k_ypass<N, double, T_D, false><<<grid_x(T_D), T_D * TPP, 0, s>>>(uh, 3, c->g, twD(c));
+    k_ypass<N, double, T_D, false><<<grid_x(T_D), T_D * TPP64, 0, s>>>(uh, 3, c->g, twD(c));
     DNS_LAUNCHED();
-    k_xplain<N, double, T_D, false, double, false, true><<<grid_x(T_D), T_D * TPP, 0, s>>>(uh, ws, 3, c->g, twD(c));
+    k_xplain<N, double, T_D, false, double, false, true><<<grid_x(T_D), T_D * TPP64, 0, s>>>(uh, ws, 3, c->g, twD(c));
     DNS_LAUNCHED();
     DNS_HIP(hipMemcpyAsync(uh, ws, 3 * sizeof(double2) * c->g.fs, hipMemcpyDeviceToDevice, s));
     int rc = state_changed(c, m);
@@ -547,19 +543,19 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
         // the adjoint's recording of this stage's u and omega (FP64, M = 1)
         double *rp = (sizeof(R) == 8 && c->rec_phys) ? c->rec_phys + (size_t)rk * 6 * g.rs : nullptr;
         if constexpr (PLANE) {
-          const dim3 gp(N, 1, M), bp(Plane<N, E_P>::THREADS);
+          const dim3 gp(N, 1, M), bp(Plane<N, E>::THREADS);
           if (rp && rk == 0)
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
           else if (rp && rk < 3)
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
           else if (rp)
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E_P, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E, REC_OK><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw, rp)));
           else if (rk == 0)
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 0, R, E><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
           else if (rk < 3)
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 1, R, E><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
           else
-            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E_P><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
+            DNS_TIMED(c, sl + 2, (k_plane<N, R, 2, R, E><<<gp, bp, 0, s>>>(W, (R *)c->us, g, invn3, tw)));
         } else if (rk == 0) {
           DNS_TIMED(c, sl + 1, (k_ypass<N, R, TY, true, 1, PIPE_Y, false, E_Y, false, true, PY><<<gy, by, 0, s>>>(W + 3 * g.wfs, 3, g, tw, g.mW)));
           if (rp)
@@ -610,11 +606,11 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // c2r of one spectral state field (state layout) into `phys`, x scale.
   int inv3_double(dns_ctx *c, const double2 *spec, double2 *tmpc, double *phys, double scale) {
     hipStream_t s = c->stream;
-    k_xplain<N, double, T_D, true, double, true><<<grid_x(T_D), T_D * TPP, 0, s>>>(spec, tmpc, 1, c->g, twD(c));
+    k_xplain<N, double, T_D, true, double, true><<<grid_x(T_D), T_D * TPP64, 0, s>>>(spec, tmpc, 1, c->g, twD(c));
     DNS_LAUNCHED();
-    k_ypass<N, double, T_D, true><<<grid_x(T_D), T_D * TPP, 0, s>>>(tmpc, 1, c->g, twD(c));
+    k_ypass<N, double, T_D, true><<<grid_x(T_D), T_D * TPP64, 0, s>>>(tmpc, 1, c->g, twD(c));
     DNS_LAUNCHED();
-    k_zc2r<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP, 0, s>>>(tmpc, phys, c->g, scale, twD(c));
+    k_zc2r<N, double, PPW64><<<N * N / PPW64, PPW64 * TPP64, 0, s>>>(tmpc, phys, c->g, scale, twD(c));
     DNS_LAUNCHED();
     return DNS_OK;
   }

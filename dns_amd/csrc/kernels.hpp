@@ -65,7 +65,7 @@ struct Geo {
 // two float pencils of 8 (six n=192 members: 5.98 -> 6.10 ms a step), and
 // blocks of five to eight waves lose anywhere (n=324 FP64 2.74 -> 4.01).
 template <int N, typename R> constexpr int z_pencils_per_block() {
-  constexpr int E = Sched<N>::E, TPP = N / E;
+  constexpr int E = Sched<N, R>::E, TPP = N / E;
   int p = TPP >= 64 ? 1 : 64 / TPP;
   while ((N * N) % p) p--;
   if (TPP < 64 && 4 * p * TPP <= 3 * 64 && (E <= 6 || (sizeof(R) == 4 && p == 1))) {
@@ -76,8 +76,8 @@ template <int N, typename R> constexpr int z_pencils_per_block() {
 }
 // Whether every pencil of a block of PPW pencils lies within one wave, so
 // that its lanes can exchange values.
-template <int N, int PPW> constexpr bool z_in_wave() {
-  constexpr int TPP = N / Sched<N>::E;
+template <int N, typename R, int PPW> constexpr bool z_in_wave() {
+  constexpr int TPP = N / Sched<N, R>::E;
   return TPP <= 64 && (PPW * TPP <= 64 || 64 % TPP == 0);
 }
 
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void k_state_rows(const T *__restrict__ src, T
 // the inverse x transform of the spectral curlX.
 // PAIR: one-dimensional launch of paired tiles (x_tile; paired_blocks).
 template <int N, typename R, int T, bool INV, int MINW = 1, int PIPE = 0, bool TRUNC = false,
-          int E = Sched<N>::E, bool CURLX = false, bool WP = false, bool PAIR = false>
+          int E = Sched<N, R>::E, bool CURLX = false, bool WP = false, bool PAIR = false>
 __global__ __launch_bounds__(T *(N / E), MINW) void k_ypass(cx<R> *__restrict__ data, int nfields, Geo g,
                                                            const cx<R> *__restrict__ tw, long mstride = 0) {
   constexpr int TPP = N / E;
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(T *(N / E), MINW) void k_ypass(cx<R> *__restrict__ 
   // the double one gains 2.84 -> 2.75 and the inverse passes 4-5%)
   constexpr bool NTL = !TRUNC || sizeof(R) == 8;
   __shared__ cx<R> lds[T * padlen<N>()];
-  __shared__ cx<R> twl[tw_size<N>()];
+  __shared__ cx<R> twl[tw_size<N, R>()];
   int bx = blockIdx.x, plane = blockIdx.y;
   if constexpr (PAIR) {
     if (!x_tile<T, R>(((TRUNC ? g.nk : N / 2 + 1) + T - 1) / T, N, bx, plane)) return;
@@ -284,11 +284,11 @@ __global__ __launch_bounds__(T *(N / E), MINW) void k_ypass(cx<R> *__restrict__ 
 // / output is in the state layout; in may equal out only when both layouts
 // are the same.  Grid (ceil(nf/T), n): blockIdx.y = j.
 template <int N, typename R, int T, bool INV, typename RI, bool SIN = false, bool SOUT = false>
-__global__ __launch_bounds__(T *(N / Sched<N>::E)) void k_xplain(const cx<RI> *in, cx<R> *out, int nfields, Geo g,
+__global__ __launch_bounds__(T *(N / Sched<N, R>::E)) void k_xplain(const cx<RI> *in, cx<R> *out, int nfields, Geo g,
                                                                   const cx<R> *__restrict__ tw) {
-  constexpr int E = Sched<N>::E, TPP = N / E;
+  constexpr int E = Sched<N, R>::E, TPP = N / E;
   __shared__ cx<R> lds[T * padlen<N>()];
-  __shared__ cx<R> twl[tw_size<N>()];
+  __shared__ cx<R> twl[tw_size<N, R>()];
   tw = stage_twiddles<N, R>(twl, tw);
   const int p = threadIdx.x % T, t = threadIdx.x / T;
   const int k = blockIdx.x * T + p;
@@ -372,13 +372,13 @@ __device__ __forceinline__ void curl_inverse_x(cx<R> (&U)[E], cx<R> (&V)[E], cx<
   }
 }
 
-template <int N, typename R, int T, bool WITH_U, typename SI, int MINW = 1, int E = Sched<N>::E>
+template <int N, typename R, int T, bool WITH_U, typename SI, int MINW = 1, int E = Sched<N, R>::E>
 __global__ __launch_bounds__(T *(N / E), MINW) void k_xinv_curl(const cx<SI> *__restrict__ uh,
                                                            cx<R> *__restrict__ W, Geo g,
                                                            const cx<R> *__restrict__ tw) {
   constexpr int TPP = N / E;
   __shared__ cx<R> lds[T * padlen<N>()];
-  __shared__ cx<R> twl[tw_size<N>()];
+  __shared__ cx<R> twl[tw_size<N, R>()];
   int bx, j;
   if (!x_tile<T, R>((N / 2 + T) / T, N, bx, j)) return;
   tw = stage_twiddles<N, R>(twl, tw);
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(T *(N / E), MINW) void k_xinv_curl(const cx<SI> *__
 // (FFTW c2r semantics).  Y == nullptr means Y = 0.  herm_load issues the
 // loads (so they can be started early), herm_combine builds the pencil.
 template <int N, typename R> struct HermRaw {
-  cx<R> x[Sched<N>::E], y[Sched<N>::E];
+  cx<R> x[(Sched<N, R>::E)], y[(Sched<N, R>::E)];
 };
 // Value of v in lane `src` of this wave (ds_bpermute; every lane active).
 template <typename R> __device__ __forceinline__ cx<R> lane_get(cx<R> v, int src) {
@@ -427,7 +427,7 @@ template <typename R> __device__ __forceinline__ cx<R> lane_get(cx<R> v, int src
 template <int N, typename R, bool IN_WAVE>
 __device__ __forceinline__ void herm_load(HermRaw<N, R> &h, const cx<R> *X, const cx<R> *Y, int t,
                                           int lim = N / 2 + 1) {
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+  constexpr int E = Sched<N, R>::E, TPP = N / E, H = N / 2;
   // Coefficients k >= lim are taken as zero and not read.
   if constexpr (IN_WAVE) {
     // Each stored element is loaded once (non-temporal): positions pos <= H
@@ -483,8 +483,8 @@ __device__ __forceinline__ void herm_load(HermRaw<N, R> &h, const cx<R> *X, cons
   }
 }
 template <int N, typename R>
-__device__ __forceinline__ void herm_combine(cx<R> (&z)[Sched<N>::E], const HermRaw<N, R> &h, int t) {
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+__device__ __forceinline__ void herm_combine(cx<R> (&z)[(Sched<N, R>::E)], const HermRaw<N, R> &h, int t) {
+  constexpr int E = Sched<N, R>::E, TPP = N / E, H = N / 2;
 #pragma unroll
   for (int c = 0; c < E; c++) {
     const int pos = t + TPP * c;
@@ -495,7 +495,7 @@ __device__ __forceinline__ void herm_combine(cx<R> (&z)[Sched<N>::E], const Herm
   }
 }
 template <int N, typename R, bool IN_WAVE>
-__device__ __forceinline__ void herm_pair(cx<R> (&z)[Sched<N>::E], const cx<R> *X, const cx<R> *Y, int t,
+__device__ __forceinline__ void herm_pair(cx<R> (&z)[(Sched<N, R>::E)], const cx<R> *X, const cx<R> *Y, int t,
                                           int lim = N / 2 + 1) {
   HermRaw<N, R> h;
   herm_load<N, R, IN_WAVE>(h, X, Y, t, lim);
@@ -505,9 +505,9 @@ __device__ __forceinline__ void herm_pair(cx<R> (&z)[Sched<N>::E], const cx<R> *
 // Split the forward FFT F of (a + i b), a and b real, into the half spectra
 // A_k = (F_k + conj F_{N-k})/2 and B_k = -i (F_k - conj F_{N-k})/2, k <= N/2.
 template <int N, typename R, class Slot>
-__device__ __forceinline__ void split_store(const cx<R> (&f)[Sched<N>::E], cx<R> *A, cx<R> *B, int t, cx<R> *lds,
+__device__ __forceinline__ void split_store(const cx<R> (&f)[(Sched<N, R>::E)], cx<R> *A, cx<R> *B, int t, cx<R> *lds,
                                             Slot slot, int lim = N / 2 + 1) {
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+  constexpr int E = Sched<N, R>::E, TPP = N / E, H = N / 2;
 #pragma unroll
   for (int c = 0; c < E; c++) lds[slot(t + TPP * c)] = f[c];
   __syncthreads();
@@ -536,7 +536,7 @@ __device__ __forceinline__ void split_store(const cx<R> (&f)[Sched<N>::E], cx<R>
 // ms).  Elsewhere the hoisted twiddles measured faster (n=512 FP64 z pass
 // 1.81 vs 2.04 ms, float 0.97 vs 1.04 ms).
 template <int N, typename R> __device__ __forceinline__ const cx<R> *z_twiddles(const cx<R> *tw) {
-  if constexpr (sizeof(R) == 8 && N / Sched<N>::E > 64) asm volatile("" : "+s"(tw));
+  if constexpr (sizeof(R) == 8 && N / Sched<N, R>::E > 64) asm volatile("" : "+s"(tw));
   return tw;
 }
 
@@ -548,9 +548,9 @@ template <int N, typename R> __device__ __forceinline__ const cx<R> *z_twiddles(
 template <int N, typename R, int MODE, typename UR, bool IW, bool REC = false>
 __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr, Geo g, R invn3,
                                      const cx<R> *__restrict__ tw, int t, cx<R> *lds, PencilSlot<N> slot,
-                                     const R (&oz0)[Sched<N>::E], R (&nz)[Sched<N>::E], const HermRaw<N, R> &h,
+                                     const R (&oz0)[(Sched<N, R>::E)], R (&nz)[(Sched<N, R>::E)], const HermRaw<N, R> &h,
                                      double *__restrict__ rec = nullptr) {
-  constexpr int E = Sched<N>::E, TPP = N / E;
+  constexpr int E = Sched<N, R>::E, TPP = N / E;
   R u[E], v[E], ww[E], ox[E], oy[E], oz[E];
   if constexpr (MODE == 0) {
     cx<R> z1[E];
@@ -631,12 +631,12 @@ __device__ __forceinline__ void zrow(cx<R> *__restrict__ w, UR *__restrict__ usr
 // REC: u and omega of every point are also stored (double) into rec, six
 // physical fields [6][n][n][n] (the adjoint's forward recomputation).
 template <int N, typename R, int PPW, int MODE, typename UR, int MINW = 1, bool REC = false>
-__global__ __launch_bounds__(PPW *(N / Sched<N>::E), MINW) void k_zfused(cx<R> *__restrict__ W, UR *__restrict__ us,
+__global__ __launch_bounds__(PPW *(N / Sched<N, R>::E), MINW) void k_zfused(cx<R> *__restrict__ W, UR *__restrict__ us,
                                                                     Geo g, R invn3,
                                                                     const cx<R> *__restrict__ tw,
                                                                     double *__restrict__ rec = nullptr) {
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
-  constexpr bool IW = z_in_wave<N, PPW>();
+  constexpr int E = Sched<N, R>::E, TPP = N / E, H = N / 2;
+  constexpr bool IW = z_in_wave<N, R, PPW>();
   __shared__ cx<R> lds[PPW * padlen<N>()];
   const int p = threadIdx.x / TPP, t = threadIdx.x % TPP;
   const long row = (long)blockIdx.x * PPW + p;
@@ -671,10 +671,10 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E), MINW) void k_zfused(cx<R> *
 // Plain r2c along z of `nfields` physical double fields into spectral
 // fields of precision R (pairs share one complex transform).
 template <int N, typename R, int PPW>
-__global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zr2c(const double *__restrict__ in, cx<R> *out,
+__global__ __launch_bounds__(PPW *(N / Sched<N, R>::E)) void k_zr2c(const double *__restrict__ in, cx<R> *out,
                                                                   int nfields, Geo g,
                                                                   const cx<R> *__restrict__ tw) {
-  constexpr int E = Sched<N>::E, TPP = N / E, H = N / 2;
+  constexpr int E = Sched<N, R>::E, TPP = N / E, H = N / 2;
   __shared__ cx<R> lds[PPW * padlen<N>()];
   const int p = threadIdx.x / TPP, t = threadIdx.x % TPP;
   const long row = (long)blockIdx.x * PPW + p;
@@ -704,16 +704,16 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zr2c(const double *_
 // Plain c2r along z of one spectral field into a physical double field,
 // multiplied by `scale` (1 for the raw transform, 1/n^3 for snapshots).
 template <int N, typename R, int PPW>
-__global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zc2r(const cx<R> *__restrict__ in,
+__global__ __launch_bounds__(PPW *(N / Sched<N, R>::E)) void k_zc2r(const cx<R> *__restrict__ in,
                                                                   double *__restrict__ out, Geo g, R scale,
                                                                   const cx<R> *__restrict__ tw) {
-  constexpr int E = Sched<N>::E, TPP = N / E;
+  constexpr int E = Sched<N, R>::E, TPP = N / E;
   __shared__ cx<R> lds[PPW * padlen<N>()];
   const int p = threadIdx.x / TPP, t = threadIdx.x % TPP;
   const long row = (long)blockIdx.x * PPW + p;
   const PencilSlot<N> slot{p * padlen<N>()};
   cx<R> z[E];
-  herm_pair<N, R, z_in_wave<N, PPW>()>(z, in + row * g.nfp, nullptr, t);
+  herm_pair<N, R, z_in_wave<N, R, PPW>()>(z, in + row * g.nfp, nullptr, t);
   fft_pencil<N, R, true>(z, t, lds, slot, tw);
 #pragma unroll
   for (int c = 0; c < E; c++) st_real<double>(out + row * N + t + TPP * c, (double)(z[c].x * scale));
@@ -744,7 +744,7 @@ __global__ __launch_bounds__(PPW *(N / Sched<N>::E)) void k_zc2r(const cx<R> *__
 // EPI selects the epilogue's batching: 0 = default (below), otherwise
 // BC = EPI & 63 positions per batch and prefetch of the next batch if
 // EPI & 64.  E = elements per thread (a multiple of the first and last radix).
-template <int N, typename R, int T, int STAGE, typename SR, int EPI = 0, int E = Sched<N>::E, bool S64 = false>
+template <int N, typename R, int T, int STAGE, typename SR, int EPI = 0, int E = Sched<N, R>::E, bool S64 = false>
 __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR> *__restrict__ uhr,
                                              double2 *__restrict__ uhn, double2 *__restrict__ acc,
                                              double2 *__restrict__ phat, Geo g, RKParams q,
@@ -1018,7 +1018,7 @@ __device__ __forceinline__ void forward_x_rk(const cx<R> *__restrict__ W, cx<SR>
 // update straight into the curl prologue and inverse x transform, saving
 // the re-read of the state.  W fields 0..2 (this stage's N) are read before
 // the same pencils' fields 0..5 are overwritten with the next partials.
-template <int N, typename R, int T, int STAGE, typename SR, int MINW = 1, int EPI = 0, int E = Sched<N>::E,
+template <int N, typename R, int T, int STAGE, typename SR, int MINW = 1, int EPI = 0, int E = Sched<N, R>::E,
           bool CX = false, bool S64 = false>
 __global__ __launch_bounds__(T *(N / E), MINW) void k_xfwd_rk_xinv(cx<R> *__restrict__ W,
                                                                        cx<SR> *__restrict__ uhr,
@@ -1027,7 +1027,7 @@ __global__ __launch_bounds__(T *(N / E), MINW) void k_xfwd_rk_xinv(cx<R> *__rest
                                                                        double2 *__restrict__ phat, Geo g,
                                                                        RKParams q, const cx<R> *__restrict__ tw) {
   __shared__ cx<R> lds[T * padlen<N>()];
-  __shared__ cx<R> twl[tw_size<N>()];
+  __shared__ cx<R> twl[tw_size<N, R>()];
   int bx, j;
   if (!x_tile<T, R>((N / 2 + T) / T, N, bx, j)) return;
   tw = stage_twiddles<N, R>(twl, tw);

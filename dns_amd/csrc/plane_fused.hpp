@@ -52,7 +52,7 @@ __global__ __launch_bounds__((Plane<N, E>::THREADS)) void k_plane(cx<R> *__restr
   using P = Plane<N, E>;
   constexpr int TPP = P::TPP, NF = P::NF, H = N / 2, NK = P::NK, C = P::C, RS = P::RS;
   __shared__ cx<R> lds[P::SLOTS];
-  __shared__ cx<R> twl[tw_size<N>()];
+  __shared__ cx<R> twl[tw_size<N, R>()];
   tw = stage_twiddles<N, R>(twl, tw);
   cx<R> *w = W + blockIdx.z * g.mW + blockIdx.x * g.wps;
   // column q of the plane, y positions ty + TPP*c

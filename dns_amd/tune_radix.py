@@ -38,23 +38,25 @@ ROOT = os.path.dirname(PKG)
 TUNE = os.path.join(PKG, "_tune")
 
 
-def table():
-    """{n: (E, radices)} of the DNS_SCHED table."""
+def table(precision="fp64"):
+    """{n: (E, radices)} that the kernels of a precision run: the DNS_SCHED
+    rows, and in the mixed forms' float kernels DNS_SCHED_FLOAT's before them."""
     with open(os.path.join(PKG, "csrc", "fft_engine.hpp")) as f:
         src = f.read()
     out = {}
-    for m in re.finditer(r"^DNS_SCHED\((\d+), (\d+), ([\d, ]+)\)", src, re.M):
-        out[int(m.group(1))] = (int(m.group(2)), tuple(int(x) for x in m.group(3).split(",")))
+    for macro in ("DNS_SCHED",) if precision == "fp64" else ("DNS_SCHED", "DNS_SCHED_FLOAT"):
+        for m in re.finditer(rf"^{macro}\((\d+), (\d+), ([\d, ]+)\)", src, re.M):
+            out[int(m.group(1))] = (int(m.group(2)), tuple(int(x) for x in m.group(3).split(",")))
     return out
 
 
 RADICES = (16, 12, 9, 8, 6, 4, 3, 2)  # dft of fft_engine.hpp
 
 
-def candidates(n):
+def candidates(n, precision="fp64"):
     """Schedules with the table's E and the fewest stages; the table's own
     schedule first, whatever its number of stages."""
-    e, cur = table()[n]
+    e, cur = table(precision)[n]
     best = []
     for stages in range(1, 12):
         for c in itertools.combinations_with_replacement(RADICES, stages):
@@ -66,8 +68,13 @@ def candidates(n):
     return e, [cur] + [c for c in best if c != cur]
 
 
-def name(n, rad):
-    return f"n{n}_" + "-".join(map(str, rad))
+def name(n, e, rad):
+    return f"n{n}_e{e}_" + "-".join(map(str, rad))
+
+
+def builds(n):
+    """(E, radices) of every candidate of either precision."""
+    return sorted({(e, c) for e, cands in (candidates(n, "fp64"), candidates(n, "mixed")) for c in cands})
 
 
 def build(sizes, jobs=8):
@@ -75,7 +82,6 @@ def build(sizes, jobs=8):
     os.makedirs(TUNE, exist_ok=True)
     work = []
     for n in sizes:
-        e, cands = candidates(n)
         # the other translation units, built once per size against a size
         # list holding n alone
         common = os.path.join(TUNE, f"n{n}_common")
@@ -91,8 +97,8 @@ def build(sizes, jobs=8):
         for fn in sorted(os.listdir(src)):
             if fn.endswith(".hip") and fn != "inst.hip":
                 work.append((os.path.join(src, fn), os.path.join(common, fn[:-4] + ".o"), []))
-        for rad in cands:
-            d = os.path.join(TUNE, name(n, rad))
+        for e, rad in builds(n):
+            d = os.path.join(TUNE, name(n, e, rad))
             os.makedirs(d, exist_ok=True)
             flags = [f"-DDNS_N={n}", f"-DDNS_SCHED_N={n}", f"-DDNS_SCHED_E={e}",
                      "-DDNS_SCHED_R=" + ",".join(map(str, rad))]
@@ -107,8 +113,8 @@ def build(sizes, jobs=8):
     for n in sizes:
         common = os.path.join(TUNE, f"n{n}_common")
         objs = [os.path.join(common, f) for f in sorted(os.listdir(common)) if f.endswith(".o")]
-        for rad in candidates(n)[1]:
-            d = os.path.join(TUNE, name(n, rad))
+        for e, rad in builds(n):
+            d = os.path.join(TUNE, name(n, e, rad))
             B._run([B.HIPCC, f"--offload-arch={B.ARCH}", "-shared", "-fPIC", "-o",
                     os.path.join(d, "libdns_hip.so"), os.path.join(d, "inst.o"), *objs])
             os.remove(os.path.join(d, "inst.o"))
@@ -116,7 +122,7 @@ def build(sizes, jobs=8):
             os.remove(f)
         shutil.rmtree(os.path.join(common, "tree"))
         shutil.rmtree(os.path.join(common, "include"))
-        print("built", n, len(candidates(n)[1]), "candidates", flush=True)
+        print("built", n, len(builds(n)), "candidates", flush=True)
 
 
 def _tgv(n):
@@ -192,22 +198,22 @@ def run(sizes, out, repeats=3, precisions=("fp64", "mixed")):
     tmp = tempfile.mkdtemp(prefix="tune_radix_")
     for n in sizes:
         steps = max(6, int(2e6 / n ** 2))
-        e, cands = candidates(n)
         for pname in precisions:
+            e, cands = candidates(n, pname)
             prec = {"fp64": 0, "mixed": 1}[pname]
             runs = {c: [] for c in cands}
             check = {}
             for rep in range(repeats):
                 order = cands[rep % len(cands):] + cands[:rep % len(cands)]
                 for rad in order:
-                    path = os.path.join(TUNE, name(n, rad), "libdns_hip.so")
-                    st_out = os.path.join(tmp, name(n, rad) + ".npy") if rep == 0 and n <= 256 else ""
+                    path = os.path.join(TUNE, name(n, e, rad), "libdns_hip.so")
+                    st_out = os.path.join(tmp, name(n, e, rad) + ".npy") if rep == 0 and n <= 256 else ""
                     p = subprocess.run([sys.executable, "-m", "dns_amd.tune_radix", "one", path, str(n), str(prec),
                                         str(steps), st_out or "-"], capture_output=True, text=True, timeout=900,
                                        cwd=ROOT)
                     line = [l for l in p.stdout.splitlines() if l.startswith("RESULT ")]
                     if p.returncode or not line:
-                        raise RuntimeError(f"candidate {name(n, rad)} {pname} failed:\n{p.stderr[-2000:]}")
+                        raise RuntimeError(f"candidate {name(n, e, rad)} {pname} failed:\n{p.stderr[-2000:]}")
                     r = json.loads(line[0][7:])
                     runs[rad].append(r["steps_per_s"])
                     if rep == 0:
@@ -253,8 +259,9 @@ def main(argv=None):
     a = ap.parse_args(argv)
     if a.what == "list":
         for n in a.sizes:
-            e, c = candidates(n)
-            print(n, e, len(c), c)
+            for pname in a.precisions.split(","):
+                e, c = candidates(n, pname)
+                print(n, pname, e, len(c), c)
     elif a.what == "build":
         build(a.sizes)
     else:

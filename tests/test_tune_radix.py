@@ -12,30 +12,33 @@ def ends_divide(e, rad):
 
 
 def test_table_covers_every_grid_size():
-    t = tune_radix.table()
-    assert sorted(t) == sorted(build.grid_sizes())
-    for n, (e, rad) in t.items():
-        assert math.prod(rad) == n, (n, rad)
-        assert ends_divide(e, rad) and set(rad) <= set(tune_radix.RADICES), (n, e, rad)
-        assert n % e == 0 and roofline.elements_per_thread(n) == e
+    for precision in ("fp64", "mixed"):
+        t = tune_radix.table(precision)
+        assert sorted(t) == sorted(build.grid_sizes())
+        for n, (e, rad) in t.items():
+            assert math.prod(rad) == n, (n, rad)
+            assert ends_divide(e, rad) and set(rad) <= set(tune_radix.RADICES), (n, e, rad)
+            assert n % e == 0 and (precision == "mixed" or roofline.elements_per_thread(n) == e)
+    assert tune_radix.table("mixed")[64] == (8, (8, 8)) and tune_radix.table()[64] == (4, (4, 4, 4))
 
 
 def test_the_table_is_the_only_one_and_every_radix_has_a_butterfly():
     """A candidate is compared with the schedule that the library runs: one
-    row a size, no second table in front of it; the tuner's radices are those
-    that the kernels implement."""
+    row a size, or one of each precision, and none that no kernel reaches; the
+    tuner's radices are those that the kernels implement."""
     with open(os.path.join(build.CSRC, "fft_engine.hpp")) as f:
         src = f.read()
-    rows = re.findall(r"^DNS_SCHED\w*\((\d+),", src, re.M)
-    assert sorted(map(int, rows)) == sorted(build.grid_sizes())
-    assert "template <int N> struct Sched : SchedTable<N> {};" in src
+    rows = re.findall(r"^(DNS_SCHED\w*)\((\d+),", src, re.M)
+    assert {m for m, _ in rows} == {"DNS_SCHED", "DNS_SCHED_FLOAT"} and len(set(rows)) == len(rows)
+    assert sorted(int(n) for m, n in rows if m == "DNS_SCHED") == sorted(build.grid_sizes())
+    assert "struct Sched : std::conditional_t<sizeof(R) == 4, SchedFloat<N>, SchedTable<N>> {};" in src
     assert sorted(tune_radix.RADICES) == sorted({int(r) for r in re.findall(r"RAD == (\d+)", src)})
 
 
 def test_candidates_are_the_fewest_stage_orderings():
-    t = tune_radix.table()
-    for n in sorted(t):
-        e, cands = tune_radix.candidates(n)
+    for n, precision in [(n, p) for n in build.grid_sizes() for p in ("fp64", "mixed")]:
+        t = tune_radix.table(precision)
+        e, cands = tune_radix.candidates(n, precision)
         assert e == t[n][0]
         assert cands[0] == t[n][1]                      # the table's own schedule first
         assert len(set(cands)) == len(cands)
@@ -51,6 +54,6 @@ def test_candidates_are_the_fewest_stage_orderings():
 
 
 def test_candidate_library_names_are_distinct():
-    e, cands = tune_radix.candidates(128)
-    names = {tune_radix.name(128, c) for c in cands}
-    assert len(names) == len(cands)
+    for n in (64, 128):
+        assert len({tune_radix.name(n, e, c) for e, c in tune_radix.builds(n)}) == len(tune_radix.builds(n))
+    assert set(tune_radix.builds(64)) >= {(4, (4, 4, 4)), (8, (8, 8))}
