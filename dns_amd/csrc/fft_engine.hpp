@@ -223,29 +223,28 @@ template <typename R, bool INV> __device__ __forceinline__ void dft4(cx<R> *a) {
   a[1] = cadd<R>(d0, d1);
   a[3] = csub<R>(d0, d1);
 }
-// (1 - c) a.  A constant's rounding error is the same in every butterfly, so
-// over three axes, and over the transforms of a step, it adds up where roundings
-// add as squares.  In double sqrt(3)/2 and sqrt(1/2) are off by 0.45 and 0.43
-// ulp (5e-17), while c = 1 - them is within 7e-18; in float by 0.26 and 0.20 ulp
-// (1.5e-8 and 1.2e-8), where c is within 6e-10 for the first and no better for
-// the second.  Error of a 3-D double transform against 80 bits, constant fused
-// with the sum -> this: n=24 2.45e-16 -> 2.27e-16, n=72 3.15 -> 2.72, n=162 3.92
-// -> 3.2, n=216 3.74 -> 3.12, n=128 3.04 -> 2.77; error of four mixed steps
-// against FP64, relative to what they change: n=24 9.7e-8 -> 7.5e-8, n=54 2.84e-7
-// -> 1.69e-7, n=162 3.77 -> 3.2, n=324 6.62 -> 5.83.  A step takes 0.1 to 1%
-// longer (FP64 n=216 2793 -> 2811 us, n=512 29.56 -> 29.63 ms; mixed n=162 760 ->
-// 765 us, n=324 4985 -> 5028).
-template <typename R> __device__ __forceinline__ cx<R> scaled_by_one_minus(cx<R> a, R c) {
-  return mk<R>(fm(-c, a.x, a.x), fm(-c, a.y, a.y));
-}
 template <typename R, bool INV> __device__ __forceinline__ void dft3(cx<R> *a) {
-  const R c = (R)0.13397459621556135323627682924706;  // 1 - sin(2 pi / 3)
   cx<R> t1 = cadd<R>(a[1], a[2]);
   const cx<R> t2 = mk<R>(fm((R)-0.5, t1.x, a[0].x), fm((R)-0.5, t1.y, a[0].y));
-  const cx<R> t3 = scaled_by_one_minus<R>(rot<R, INV>(csub<R>(a[1], a[2])), c);
+  const cx<R> d = rot<R, INV>(csub<R>(a[1], a[2]));
   a[0] = cadd<R>(a[0], t1);
-  a[1] = cadd<R>(t2, t3);
-  a[2] = csub<R>(t2, t3);
+  if constexpr (sizeof(R) == 8) {
+    const R s3 = (R)0.86602540378443864676372317075294;  // sin(2 pi / 3)
+    a[1] = mk<R>(fm(s3, d.x, t2.x), fm(s3, d.y, t2.y));
+    a[2] = mk<R>(fm(-s3, d.x, t2.x), fm(-s3, d.y, t2.y));
+  } else {
+    // As 1 - c in float: a constant's rounding error is the same in every
+    // butterfly, so over three axes and the transforms of a step it adds up
+    // where roundings add as squares; sin(2 pi / 3) is off by 0.26 ulp (1.5e-8),
+    // c is within 6e-10.  Error of four mixed steps against FP64, relative to
+    // what they change, constant fused with the sum -> this: n=24 9.7e-8 ->
+    // 7.5e-8, n=54 2.84e-7 -> 1.69e-7, n=162 3.77 -> 3.2, n=324 6.62 -> 5.83; a
+    // step takes 0.1 to 1% longer (n=162 760 -> 765 us, n=324 4985 -> 5028).
+    const R c = (R)0.13397459621556135323627682924706;
+    const cx<R> t3 = mk<R>(fm(-c, d.x, d.x), fm(-c, d.y, d.y));
+    a[1] = cadd<R>(t2, t3);
+    a[2] = csub<R>(t2, t3);
+  }
 }
 template <typename R, bool INV> __device__ __forceinline__ void dft8(cx<R> *a) {
   const R h = (R)0.70710678118654752440084436210485;  // 1/sqrt(2)
@@ -268,19 +267,10 @@ template <typename R, bool INV> __device__ __forceinline__ void dft8(cx<R> *a) {
   dft4<R, INV>(s);
   const cx<R> s0 = cadd<R>(d[0], d[2]), d0 = csub<R>(d[0], d[2]);
   const cx<R> s1 = cadd<R>(d[1], d[3]), d1 = rot<R, INV>(csub<R>(d[1], d[3]));
-  if constexpr (sizeof(R) == 8) {
-    const R c = (R)0.29289321881345247559915563789515;  // 1 - h
-    const cx<R> hs = scaled_by_one_minus<R>(s1, c), hd = scaled_by_one_minus<R>(d1, c);
-    a[1] = cadd<R>(s0, hs);
-    a[3] = cadd<R>(d0, hd);
-    a[5] = csub<R>(s0, hs);
-    a[7] = csub<R>(d0, hd);
-  } else {
-    a[1] = mk<R>(fm(h, s1.x, s0.x), fm(h, s1.y, s0.y));
-    a[3] = mk<R>(fm(h, d1.x, d0.x), fm(h, d1.y, d0.y));
-    a[5] = mk<R>(fm(-h, s1.x, s0.x), fm(-h, s1.y, s0.y));
-    a[7] = mk<R>(fm(-h, d1.x, d0.x), fm(-h, d1.y, d0.y));
-  }
+  a[1] = mk<R>(fm(h, s1.x, s0.x), fm(h, s1.y, s0.y));
+  a[3] = mk<R>(fm(h, d1.x, d0.x), fm(h, d1.y, d0.y));
+  a[5] = mk<R>(fm(-h, s1.x, s0.x), fm(-h, s1.y, s0.y));
+  a[7] = mk<R>(fm(-h, d1.x, d0.x), fm(-h, d1.y, d0.y));
 #pragma unroll
   for (int p = 0; p < 4; p++) a[2 * p] = s[p];
 }

@@ -1,0 +1,38 @@
+"""Mixed steps against FP64 steps: the rounding error stays that of the schedules
+of radices 4, 3 and 2 that these grids had before, measured on the same inputs.
+Other orders of the radices and a second stage of float twiddles had raised it by
+up to 8% through the rounding of their constants, which is alike in every
+butterfly and axis.  2% for the sampling of the fields."""
+import numpy as np
+import pytest
+
+import dns_amd
+from conftest import wavenumbers
+
+pytestmark = pytest.mark.gpu
+
+# relative to what four steps change, mean of six fields
+FORMER = {24: 9.305e-8, 54: 3.186e-7, 64: 1.667e-7}
+
+
+@pytest.mark.parametrize("n", sorted(FORMER))
+def test_mixed_step_error_is_no_larger_than_before(n):
+    print(f"mixed step error n={n}", flush=True)
+    kx, ky, kz = wavenumbers(n)
+    kk = kx * kx + ky * ky + kz * kz
+    errors = []
+    for q in range(6):
+        rng = np.random.default_rng(100 * n + q)
+        a = np.stack([np.fft.rfftn(rng.standard_normal((n, n, n))) for _ in range(3)])
+        a *= np.sqrt(kk) * np.exp(-kk / (n / 8) ** 2)
+        a *= n ** 3 / np.sqrt(2 * np.sum(np.abs(a) ** 2))
+        out = {}
+        for precision in ("fp64", "mixed"):
+            with dns_amd.Solver(n, 1 / 400, 0.1 / n, precision) as s:
+                s.load_velocity(np.zeros((3, n, n, n)))
+                s.set_spectral(a)
+                s.step(4)
+                out[precision] = s.get_spectral()
+        errors.append(np.linalg.norm(out["mixed"] - out["fp64"]) / np.linalg.norm(out["fp64"] - a))
+    print(f"  {np.mean(errors):.3e}", flush=True)
+    assert np.mean(errors) <= 1.02 * FORMER[n]
