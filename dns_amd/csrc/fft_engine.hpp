@@ -224,27 +224,13 @@ template <typename R, bool INV> __device__ __forceinline__ void dft4(cx<R> *a) {
   a[3] = csub<R>(d0, d1);
 }
 template <typename R, bool INV> __device__ __forceinline__ void dft3(cx<R> *a) {
+  const R s3 = (R)0.86602540378443864676372317075294;  // sin(2 pi / 3)
   cx<R> t1 = cadd<R>(a[1], a[2]);
   const cx<R> t2 = mk<R>(fm((R)-0.5, t1.x, a[0].x), fm((R)-0.5, t1.y, a[0].y));
   const cx<R> d = rot<R, INV>(csub<R>(a[1], a[2]));
   a[0] = cadd<R>(a[0], t1);
-  if constexpr (sizeof(R) == 8) {
-    const R s3 = (R)0.86602540378443864676372317075294;  // sin(2 pi / 3)
-    a[1] = mk<R>(fm(s3, d.x, t2.x), fm(s3, d.y, t2.y));
-    a[2] = mk<R>(fm(-s3, d.x, t2.x), fm(-s3, d.y, t2.y));
-  } else {
-    // As 1 - c in float: a constant's rounding error is the same in every
-    // butterfly, so over three axes and the transforms of a step it adds up
-    // where roundings add as squares; sin(2 pi / 3) is off by 0.26 ulp (1.5e-8),
-    // c is within 6e-10.  Error of four mixed steps against FP64, relative to
-    // what they change, constant fused with the sum -> this: n=24 9.7e-8 ->
-    // 7.5e-8, n=54 2.84e-7 -> 1.69e-7, n=162 3.77 -> 3.2, n=324 6.62 -> 5.83; a
-    // step takes 0.1 to 1% longer (n=162 760 -> 765 us, n=324 4985 -> 5028).
-    const R c = (R)0.13397459621556135323627682924706;
-    const cx<R> t3 = mk<R>(fm(-c, d.x, d.x), fm(-c, d.y, d.y));
-    a[1] = cadd<R>(t2, t3);
-    a[2] = csub<R>(t2, t3);
-  }
+  a[1] = mk<R>(fm(s3, d.x, t2.x), fm(s3, d.y, t2.y));
+  a[2] = mk<R>(fm(-s3, d.x, t2.x), fm(-s3, d.y, t2.y));
 }
 template <typename R, bool INV> __device__ __forceinline__ void dft8(cx<R> *a) {
   const R h = (R)0.70710678118654752440084436210485;  // 1/sqrt(2)
