@@ -242,8 +242,9 @@ template <int N, typename R, typename SR, bool S64 = false> struct Engine final 
   // chip either way, gain as well, from 2 to 48 members: FP64 n=48 six 296 ->
   // 284, 48 of them 1816 -> 1509; n=24 133 -> 93 and 340 -> 229; mixed n=72 478
   // -> 404 and 3224 -> 2776.
-  static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72);
-  static_assert(!PLANE || Plane<N, E>::THREADS <= 1024, "a plane's columns fit a block");
+  // Not where a schedule gives a plane more threads than a block holds (float
+  // n=64 with 4 elements each, a candidate of the tuner).
+  static constexpr bool PLANE = N <= (sizeof(R) == 8 ? 48 : 72) && Plane<N, E>::THREADS <= 1024;
   // y passes: double grids whose pencils need more than 64 threads (n=864 to
   // 1024) take twice the elements per thread (n=1024: 16), keeping 8-column
   // tiles in 512 threads (n=1024: inverse 25.0 -> 22.5 ms, forward 7.7 -> 5.7 ms).

@@ -17,7 +17,7 @@ def _source(name):
 
 def test_thresholds_are_the_kernels():
     first, = re.findall(r"constexpr bool SKIP = N >= (\d+);", _source("kernels.hpp"))
-    d, f = re.findall(r"constexpr bool PLANE = N <= \(sizeof\(R\) == 8 \? (\d+) : (\d+)\);", _source("engine.hpp"))[0]
+    d, f = re.findall(r"constexpr bool PLANE = N <= \(sizeof\(R\) == 8 \? (\d+) : (\d+)\)", _source("engine.hpp"))[0]
     for n in build.grid_sizes():
         assert roofline.stores_all_modes(n) == (n < int(first))
         assert roofline.plane_fused(n, "fp64") == (n <= int(d))

@@ -4,6 +4,8 @@ import math
 import os
 import re
 
+import pytest
+
 from dns_amd import build, roofline, tune_radix
 
 
@@ -57,3 +59,10 @@ def test_candidate_library_names_are_distinct():
     for n in (64, 128):
         assert len({tune_radix.name(n, e, c) for e, c in tune_radix.builds(n)}) == len(tune_radix.builds(n))
     assert set(tune_radix.builds(64)) >= {(4, (4, 4, 4)), (8, (8, 8))}
+
+
+@pytest.mark.parametrize("e,rad", tune_radix.builds(64))
+def test_every_candidate_of_a_size_with_two_schedules_compiles(e, rad):
+    """A candidate build replaces the schedules of both precisions."""
+    flags = ["-DDNS_N=64", "-DDNS_SCHED_N=64", f"-DDNS_SCHED_E={e}", "-DDNS_SCHED_R=" + ",".join(map(str, rad))]
+    build._run([build.HIPCC, *build.HIP_FLAGS, *flags, "-fsyntax-only", os.path.join(build.CSRC, "inst.hip")])
